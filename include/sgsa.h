@@ -88,7 +88,7 @@ int sgsa_chunk_fwd(int dtype, int B, int T, int H, int D, int chunk_size,
  * input dtype; dbeta, dgamma, dalpha [B,T,H] fp32; d_final_state and
  * d_initial_state [B,H,D,D] fp32 (either may be NULL).  The sparse write's
  * inputs and gradients are given together or not at all.  Needs
- * sgsa_chunk_bwd_workspace_size() bytes (about 0.8 MB per 64-token chunk and
+ * sgsa_chunk_bwd_workspace_size() bytes (about 0.36 MB per 64-token chunk and
  * head with the sparse write). */
 int sgsa_chunk_bwd_workspace_size(int B, int T, int H, int D, int has_sparse, size_t* bytes);
 int sgsa_chunk_bwd(int dtype, int B, int T, int H, int D,

@@ -77,7 +77,7 @@ LayerWs layer_ws(int dtype, int B, int T, int H, int D, int top_k) {
   w.al = off; off = align_up(off + (size_t)B * T * H * 4);
   w.misc = off; off = align_up(off + 256);
   w.topk = off; off = align_up(off + sgsa::topk_workspace_bytes(B, T, H));
-  w.chunk = off; off = align_up(off + sgsa::chunk_workspace_bytes(B, T, H, 1));
+  w.chunk = off; off = align_up(off + sgsa::chunk_workspace_bytes(B, T, H, D, 1));
   w.total = off + kAlign;
   return w;
 }
@@ -116,7 +116,7 @@ extern "C" {
 int sgsa_chunk_fwd_workspace_size(int B, int T, int H, int D, int has_sparse, size_t* bytes) {
   REQUIRE(bytes);
   if (int s = check_dims(B, T, H, D)) return s;
-  *bytes = sgsa::chunk_workspace_bytes(B, T, H, has_sparse ? 1 : 0);
+  *bytes = sgsa::chunk_workspace_bytes(B, T, H, D, has_sparse ? 1 : 0);
   return SGSA_OK;
 }
 
@@ -130,7 +130,7 @@ int sgsa_chunk_fwd(int dtype, int B, int T, int H, int D, int chunk_size, const 
   REQUIRE(q); REQUIRE(k); REQUIRE(v); REQUIRE(beta); REQUIRE(gamma); REQUIRE(out); REQUIRE(workspace);
   const int nsp = (sparse_k != nullptr) + (sparse_v != nullptr) + (alpha != nullptr);
   if (nsp != 0 && nsp != 3) return fail(SGSA_ERR_INVALID_ARG, "sparse_k, sparse_v and alpha must be given together");
-  const size_t need = sgsa::chunk_workspace_bytes(B, T, H, nsp == 3);
+  const size_t need = sgsa::chunk_workspace_bytes(B, T, H, D, nsp == 3);
   if (workspace_bytes < need) return fail(SGSA_ERR_WORKSPACE, "workspace %zu < %zu bytes", workspace_bytes, need);
   sgsa::ChunkArgs a{};
   a.dtype = dtype; a.B = B; a.T = T; a.H = H; a.D = D;
@@ -145,7 +145,7 @@ int sgsa_chunk_fwd(int dtype, int B, int T, int H, int D, int chunk_size, const 
 int sgsa_chunk_bwd_workspace_size(int B, int T, int H, int D, int has_sparse, size_t* bytes) {
   if (int s = check_dims(B, T, H, D)) return s;
   REQUIRE(bytes);
-  *bytes = sgsa::chunk_bwd_workspace_bytes(B, T, H, has_sparse != 0);
+  *bytes = sgsa::chunk_bwd_workspace_bytes(B, T, H, D, has_sparse != 0);
   return SGSA_OK;
 }
 
@@ -163,7 +163,7 @@ int sgsa_chunk_bwd(int dtype, int B, int T, int H, int D, const void* q, const v
   if (nsp == 3 && (dsparse_k == nullptr || dsparse_v == nullptr || dalpha == nullptr))
     return fail(SGSA_ERR_INVALID_ARG, "the sparse write needs dsparse_k, dsparse_v and dalpha outputs");
   if ((long)T * H > 0x7fffffffL) return fail(SGSA_ERR_UNSUPPORTED, "T*H too large");
-  const size_t need = sgsa::chunk_bwd_workspace_bytes(B, T, H, nsp == 3);
+  const size_t need = sgsa::chunk_bwd_workspace_bytes(B, T, H, D, nsp == 3);
   if (workspace_bytes < need) return fail(SGSA_ERR_WORKSPACE, "workspace %zu < %zu bytes", workspace_bytes, need);
   sgsa::ChunkBwdArgs a{};
   a.f.dtype = dtype; a.f.B = B; a.f.T = T; a.f.H = H; a.f.D = D;

@@ -27,16 +27,22 @@ struct ChunkArgs {
   void* workspace;
 };
 
-size_t chunk_workspace_bytes(int B, int T, int H, int has_sparse);   // covers both paths
+size_t chunk_workspace_bytes(int B, int T, int H, int D, int has_sparse);   // covers both paths
 size_t chunk_bf16_workspace_bytes(int B, int T, int H, int has_sparse);
 hipError_t launch_chunk_fwd(const ChunkArgs& a, hipStream_t st);
 hipError_t launch_chunk_bf16(const ChunkArgs& a, hipStream_t st);
-// The fp32 chunk path's per-chunk intermediates for the backward (chunk.hip): per
-// (b*H + h, chunk) W, U [M][128], the log-decay prefix [64] and A [M][M]
-// (M = 128 with the sparse write, else 64).
-hipError_t launch_chunk_intra(const ChunkArgs& a, float* W, float* U, float* lgd, float* A, hipStream_t st);
-// The same operands for bf16 inputs from the forward's K3 (chunk_inv_bf16 in its backward form).
-hipError_t launch_chunk_intra_bf16(const ChunkArgs& a, float* W, float* U, float* lgd, float* A, hipStream_t st);
+// Head dimension the fp32 chunk kernels run at (their tiles and workspace rows are padded to it).
+inline int chunk_f32_dp(int D) { return D <= 64 ? 64 : 128; }
+// The fp32 chunk form's first stages, for bf16 or fp32 inputs (chunk.hip), per (b*H + h, chunk):
+// the log-decay prefix [64], the lower 16x16 tiles of the WY inverse A [M][M] ([NTL][16][16];
+// M = 128 with the sparse write, else 64), the chunk's affine state map Phi, Pm [DP][DP] and the
+// chunk-start state Hs [DP][DP] (DP = chunk_f32_dp(D)); ht [B,H,D,D] the final state or nullptr.
+void launch_chunk_states(const ChunkArgs& a, float* lgd, float* A, float* Phi, float* Pm, float* Hs, float* ht,
+                         hipStream_t st);
+// x <- phi_c x + y_c over a head's NT chunks (tr: phi_c^T, from the last chunk): x before each
+// step in out, all [BH][NT][dp][dp]; init and last [BH][D][D] or nullptr (chunk.hip).
+void launch_chunk_scan(int dp, bool tr, const float* phi, const float* y, int BH, int NT, const float* init, int D,
+                       float* out, float* last, hipStream_t st);
 
 // Backward of chunk_sgsa (chunk_bwd.hip).
 struct ChunkBwdArgs {
@@ -48,7 +54,7 @@ struct ChunkBwdArgs {
   float* d_initial_state;       // [B,H,D,D] fp32 or nullptr
   void* workspace;
 };
-size_t chunk_bwd_workspace_bytes(int B, int T, int H, int has_sparse);
+size_t chunk_bwd_workspace_bytes(int B, int T, int H, int D, int has_sparse);
 hipError_t launch_chunk_bwd(const ChunkBwdArgs& a, hipStream_t st);
 
 struct RecurrentArgs {

@@ -239,15 +239,18 @@ int score_topk_launch(const sgsa::TopkArgs& a0, int sorted, void* workspace, siz
                       hipStream_t st) {
   sgsa::TopkArgs a = a0;
   a.workspace = workspace;
+  a.sort = sorted;
+  bool done = false;   // the launch sorted the rows
   const size_t base_ws = (sgsa::topk_workspace_bytes(a.B, a.Tq, a.H) + 255) & ~(size_t)255;
   const size_t rows_ws = sgsa::topk_rows_bytes(a);
   if (rows_ws > 0 && workspace_bytes >= base_ws + rows_ws && ((uintptr_t)workspace & 255u) == 0) {
     float* sbuf = reinterpret_cast<float*>(static_cast<char*>(workspace) + base_ws);
     if (int s = hip_status(sgsa::launch_score_topk_rows(a, sbuf, st), "sgsa_score_topk (few rows)")) return s;
-  } else if (int s = hip_status(sgsa::launch_score_topk(a, st), "sgsa_score_topk")) {
-    return s;
+  } else {
+    if (int s = hip_status(sgsa::launch_score_topk(a, st), "sgsa_score_topk")) return s;
+    done = sgsa::topk_buf_sorts(a);
   }
-  if (sorted)
+  if (sorted && !done)
     return hip_status(sgsa::launch_sort_rows(a.indices, a.scores, (long)a.B * a.H * a.Tq, a.top_k, a.counts, st),
                       "sgsa_score_topk(sort)");
   return SGSA_OK;
@@ -387,9 +390,10 @@ int sgsa_score_topk_masked(int dtype, int B, int Tq, int Tk, int H, int D, int t
                                      m.compacted ? m.kc : k, indices, scores, top2, counts, nullptr);
   a.row_nv = m.nv;
   a.row_kq = m.kq;
+  a.sort = sorted;
   a.workspace = base + align_up(sgsa::mask_workspace_bytes(dtype, B, Tq, Tk, H, D, m.compacted));
   if (int s = hip_status(sgsa::launch_score_topk(a, st), "sgsa_score_topk_masked")) return s;
-  if (sorted) {   // (score desc, index asc): the compaction keeps the index order
+  if (sorted && !sgsa::topk_buf_sorts(a)) {   // (score desc, index asc): the compaction keeps the index order
     if (int s = hip_status(sgsa::launch_sort_rows(indices, scores, (long)B * H * Tq, top_k, counts, st),
                            "sgsa_score_topk_masked (sort)"))
       return s;

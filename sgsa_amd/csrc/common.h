@@ -35,6 +35,11 @@ template <> struct elem<bf16_t> {
   __device__ __forceinline__ static void store(bf16_t* p, long i, float v) { p[i].bits = f32_to_bf16(v); }
 };
 
+// The unsigned (bf16) or plain (fp32) element type of raw tiles.
+template <typename X> struct elem_bits;
+template <> struct elem_bits<float> { typedef float T; };
+template <> struct elem_bits<bf16_t> { typedef uint16_t T; };
+
 template <typename X>
 __device__ __forceinline__ float ld(const X* p, long i) { return elem<X>::load(p, i); }
 template <typename X>

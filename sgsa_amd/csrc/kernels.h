@@ -94,6 +94,7 @@ struct TopkArgs {
   float* scores;      // [B,H,Tq,top_k]
   float* top2;        // [B,H,Tq,2] or nullptr
   int32_t* counts;    // [B,H,Tq] valid selected slots, or nullptr
+  int sort;           // the caller wants (score desc, index asc); topk_buf_sorts says whether the launch does it
   int32_t* split;     // [B,H,Tq] length of the leading ascending-index run, or nullptr
   float* dump;        // score-dump mode: [B,H,dump_rows,Tk]; nullptr = select mode
   int dump_row0, dump_rows;
@@ -136,6 +137,14 @@ hipError_t launch_mask_finish(const MaskArgs& m, int32_t* indices, float* scores
                               const int32_t* counts, int32_t* fill, hipStream_t st);
 
 constexpr int TOPK_CAP = 512;   // collected threshold-bin candidates per row
+
+// Score-buffer form of the row lists (topk_buf.hip): up to BUF_MAXK keys; buf the candidate
+// lists' part of topk_workspace_bytes().
+constexpr int BUF_MAXK = 8192;
+constexpr int BUF_SORT = 512;   // rows of up to this many slots leave the select sorted, if asked
+bool topk_buf_fits(const TopkArgs& a);
+inline bool topk_buf_sorts(const TopkArgs& a) { return topk_buf_fits(a) && a.top_k <= BUF_SORT; }
+hipError_t launch_score_topk_buf(const TopkArgs& a, float* buf, hipStream_t st);
 
 // Few-row form of the select (topk_rows.hip): bf16, D % 32 == 0, at most
 // TR_MAX_TQ query rows per (b, h), TR_MAX_ROWS rows and TR_MAXK keys.  Extra

@@ -33,13 +33,6 @@ __device__ __host__ constexpr int tri(int I, int J) { return I * (I + 1) / 2 + J
 template <int M> __device__ __forceinline__ int samp_t(int i) { return M == 2 * L ? (i >> 1) : i; }
 template <int M> __device__ __forceinline__ int samp_r(int i) { return M == 2 * L ? (i & 1) : 0; }
 
-// Four consecutive elements as fp32.
-__device__ __forceinline__ f4 vload4(const float* p) { return *reinterpret_cast<const f4*>(p); }
-__device__ __forceinline__ f4 vload4(const bf16_t* p) {
-  const uint2 u = *reinterpret_cast<const uint2*>(p);
-  return f4{__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16),
-            __uint_as_float(u.y & 0xffff0000u)};
-}
 __device__ __forceinline__ void vstore4(float* p, f4 v) { *reinterpret_cast<f4*>(p) = v; }
 __device__ __forceinline__ void vstore4(bf16_t* p, f4 v) {
   *reinterpret_cast<uint2*>(p) = make_uint2((uint32_t)f32_to_bf16(v[0]) | ((uint32_t)f32_to_bf16(v[1]) << 16),

@@ -45,6 +45,14 @@ __device__ __forceinline__ float ld(const X* p, long i) { return elem<X>::load(p
 template <typename X>
 __device__ __forceinline__ void st(X* p, long i, float v) { elem<X>::store(p, i, v); }
 
+// Four consecutive elements as fp32.
+__device__ __forceinline__ f4 vload4(const float* p) { return *reinterpret_cast<const f4*>(p); }
+__device__ __forceinline__ f4 vload4(const bf16_t* p) {
+  const uint2 u = *reinterpret_cast<const uint2*>(p);
+  return f4{__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16),
+            __uint_as_float(u.y & 0xffff0000u)};
+}
+
 // Order-preserving map fp32 -> uint32 (larger float => larger key).  -0.0 is
 // folded onto +0.0 first so the two compare equal, as IEEE comparison does.
 __device__ __forceinline__ uint32_t f32_order_key(float f) {

@@ -9,11 +9,26 @@
 
 namespace sgsa {
 
+// The sums over the 128 rows of a column, in one order wherever K6 runs: chains of 16 rows in
+// ascending order, c_0 .. c_7, then ((c0 + c1) + (c2 + c3)) + ((c4 + c5) + (c6 + c7)).  A thread
+// holding several chains adds its own first; T one-token calls then equal one T-token call, and
+// every split of the columns any other, bit for bit.
+template <int N>
+__device__ __forceinline__ float sum_chains(const float (&c)[N]) {
+  static_assert(N == 1 || N == 2 || N == 4 || N == 8, "a power of two, at most the 8 chains of 128 rows");
+  if constexpr (N == 1) return c[0];
+  else if constexpr (N == 2) return c[0] + c[1];
+  else if constexpr (N == 4) return (c[0] + c[1]) + (c[2] + c[3]);
+  else return ((c[0] + c[1]) + (c[2] + c[3])) + ((c[4] + c[5]) + (c[6] + c[7]));
+}
+
 template <typename X, bool SP, int CS>
 __device__ __forceinline__ void recurrent_body(const RecurrentArgs& a) {
   constexpr int RC = 128 / CS;     // columns per block
   constexpr int NG = 256 / RC;     // row groups
   constexpr int RR = 128 / NG;     // rows per thread
+  constexpr int NC = RR / 16;      // 16-row chains per thread
+  static_assert(RR % 16 == 0, "whole chains");
   __shared__ float vq[128], vk[128], vkh[128];   // q, k, kh of the current token (all rows)
   __shared__ float vv[RC], vvh[RC];              // v, vh (this tile's columns)
   __shared__ float part[3][NG][RC];              // partial base^T k, base^T kh, S^T q per row group
@@ -79,39 +94,45 @@ __device__ __forceinline__ void recurrent_body(const RecurrentArgs& a) {
     if (t + 1 < T) fetch(t + 1);
     const float gam = scal[1];
     // base = gamma S; predictions base^T k and base^T kh over this thread's rows
-    float pk = 0.f, ph = 0.f;
+    float pk[NC], ph[NC];
 #pragma unroll
-    for (int r = 0; r < RR; ++r) {
-      S[r] *= gam;
-      pk = fmaf(S[r], vk[RR * g + r], pk);
-      if constexpr (SP) ph = fmaf(S[r], vkh[RR * g + r], ph);
+    for (int c = 0; c < NC; ++c) {
+      pk[c] = ph[c] = 0.f;
+#pragma unroll
+      for (int r = 16 * c; r < 16 * c + 16; ++r) {
+        S[r] *= gam;
+        pk[c] = fmaf(S[r], vk[RR * g + r], pk[c]);
+        if constexpr (SP) ph[c] = fmaf(S[r], vkh[RR * g + r], ph[c]);
+      }
     }
-    part[0][g][jl] = pk;
-    if constexpr (SP) part[1][g][jl] = ph;
+    part[0][g][jl] = sum_chains(pk);
+    if constexpr (SP) part[1][g][jl] = sum_chains(ph);
     __syncthreads();
-    float sk_ = 0.f, sh_ = 0.f;
+    auto total = [&](int n) __attribute__((always_inline)) {
+      float x[NG];
 #pragma unroll
-    for (int u = 0; u < NG; ++u) {
-      sk_ += part[0][u][jl];
-      if constexpr (SP) sh_ += part[1][u][jl];
-    }
-    const float dl = scal[0] * (vv[jl] - sk_);
-    const float ds = SP ? scal[2] * (vvh[jl] - sh_) : 0.f;
+      for (int u = 0; u < NG; ++u) x[u] = part[n][u][jl];
+      return sum_chains(x);
+    };
+    const float dl = scal[0] * (vv[jl] - total(0));
+    const float ds = SP ? scal[2] * (vvh[jl] - total(1)) : 0.f;
     // rank-1 writes, then the readout o = S^T q
-    float po = 0.f;
+    float po[NC];
 #pragma unroll
-    for (int r = 0; r < RR; ++r) {
-      const int i = RR * g + r;
-      S[r] = fmaf(vk[i], dl, S[r]);
-      if constexpr (SP) S[r] = fmaf(vkh[i], ds, S[r]);
-      po = fmaf(S[r], vq[i], po);
+    for (int c = 0; c < NC; ++c) {
+      po[c] = 0.f;
+#pragma unroll
+      for (int r = 16 * c; r < 16 * c + 16; ++r) {
+        const int i = RR * g + r;
+        S[r] = fmaf(vk[i], dl, S[r]);
+        if constexpr (SP) S[r] = fmaf(vkh[i], ds, S[r]);
+        po[c] = fmaf(S[r], vq[i], po[c]);
+      }
     }
-    part[2][g][jl] = po;
+    part[2][g][jl] = sum_chains(po);
     __syncthreads();
     if (g == 0 && colv) {
-      float o = 0.f;
-#pragma unroll
-      for (int u = 0; u < NG; ++u) o += part[2][u][jl];
+      const float o = total(2);
       st(reinterpret_cast<X*>(a.out), ((long)(b * T + t) * H + h) * D + j, o);
     }
   }

@@ -30,6 +30,7 @@
 
 #include "common.h"
 #include "kernels.h"
+#include "wave_sort.h"
 
 namespace sgsa {
 
@@ -543,9 +544,9 @@ __global__ __launch_bounds__(256, 2) void block_max_reg_kernel(BlockArgs a, floa
   const int D = NKS * 32, T = a.T, H = a.H, bs = a.bs, nb = a.nb;
   const int nrb = (T + QR - 1) / QR;
   // grid (B*H, row blocks): consecutive workgroups take different heads, so the XCDs they are dealt
-  // to in turn each see a few heads' keys in their L2; the latest (heaviest) row blocks go first
+  // to in turn each see a few heads' keys in their L2
   const int bh = blockIdx.x, b = bh / H, h = bh % H;
-  const int r0 = (nrb - 1 - (int)blockIdx.y) * QR;
+  const int r0 = (nrb - 1 - causal_block((int)blockIdx.y, nrb, (int)gridDim.x)) * QR;
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, lg = lane >> 4;
   const uint16_t* Q = reinterpret_cast<const uint16_t*>(a.q);
@@ -843,7 +844,12 @@ __global__ __launch_bounds__(64) void block_cand_kernel(BlockArgs a, float mscal
   const X* Q = reinterpret_cast<const X*>(a.q);
   const X* K = reinterpret_cast<const X*>(a.k);
 
-  for (int d = lane; d < D; d += 64) qrow[d] = ld(Q, ((long)(b * T + t) * H + h) * D + d);
+  // the position's candidate counts over the batch and heads, for k_q below
+  int mcl = 0;
+  if constexpr (TOKEN)
+    for (int e = lane; e < a.B * a.H; e += 64) mcl = max(mcl, a.ncand[(long)e * T + t]);
+  if constexpr (!MF)
+    for (int d = lane; d < D; d += 64) qrow[d] = ld(Q, ((long)(b * T + t) * H + h) * D + d);
   // candidates of kept block s: its keys <= lim (with a mask, its valid ones)
   int run = 0;
   for (int s0 = 0; s0 < kqb; s0 += 64) {
@@ -977,45 +983,74 @@ __global__ __launch_bounds__(64) void block_cand_kernel(BlockArgs a, float mscal
     return;
   }
 
-  int npad = 1;
-  while (npad < ncand) npad <<= 1;
-  for (int c = ncand + lane; c < npad; c += 64) keys[c] = ~0ull;
-  wave_sync_lds();
-  for (int span = 2; span <= npad; span <<= 1) {
-    for (int j = span >> 1; j > 0; j >>= 1) {
-      for (int i = lane; i < npad; i += 64) {
-        const int p = i ^ j;
-        if (p > i) {
-          const uint64_t x = keys[i], y = keys[p];
-          if ((x > y) == ((i & span) == 0)) {
-            keys[i] = y;
-            keys[p] = x;
-          }
-        }
-      }
-      wave_sync_lds();
-    }
-  }
-
-  int mc = 1;
-  for (int e = lane; e < a.B * a.H; e += 64) mc = max(mc, a.ncand[(long)e * T + t]);
+  // the candidates by (score desc, key asc): up to 512 in registers, more in LDS (131072 rows of 64
+  // candidates: 287 us all in LDS, 281; the reads of the candidates' keys, 2.1 GB, bound both)
+  int mc = max(1, mcl);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) mc = max(mc, __shfl_xor(mc, o, 64));
   const int kk = a.kk, kq = min(kk, mc), nv = min(ncand, kq);
   int32_t* oi = a.slot_idx + row * kk;
   float* os = a.slot_sc + row * kk;
   uint8_t* ov = a.slot_valid + row * kk;
-  for (int i = lane; i < kk; i += 64) {
-    if (i < nv) {
-      const uint64_t x = keys[i];
-      oi[i] = (int)(uint32_t)x;
-      os[i] = key_to_f32(~(uint32_t)(x >> 32));
-      ov[i] = 1;
-    } else if (i >= kq) {
-      oi[i] = 0;
-      os[i] = -FLT_MAX;
-      ov[i] = 0;
+  float top0 = -FLT_MAX, top1 = -FLT_MAX;
+  auto put = [&](int i, uint32_t key, uint32_t ord) __attribute__((always_inline)) {
+    oi[i] = (int)key;
+    os[i] = key_to_f32(ord);
+    ov[i] = 1;
+  };
+  wave_sync_lds();
+  if (ncand <= 512) {
+    auto sort = [&](auto ns) __attribute__((always_inline)) {
+      constexpr int NS = decltype(ns)::value;
+      uint32_t hi[NS], lo[NS];
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        const int c = 64 * s + lane;
+        const uint64_t x = c < ncand ? keys[c] : ~0ull;   // padding sorts last
+        hi[s] = ~(uint32_t)(x >> 32);
+        lo[s] = ~(uint32_t)x;
+      }
+      wave_sort_desc<NS>(hi, lo, lane);
+#pragma unroll
+      for (int s = 0; s < NS; ++s)
+        if (NS * lane + s < nv) put(NS * lane + s, ~lo[s], hi[s]);
+      const uint32_t h0 = (uint32_t)__builtin_amdgcn_readlane((int)hi[0], 0);
+      const uint32_t h1 = (uint32_t)__builtin_amdgcn_readlane((int)hi[NS > 1 ? 1 : 0], NS > 1 ? 0 : 1);
+      if (nv >= 1) top0 = key_to_f32(h0);
+      if (nv >= 2) top1 = key_to_f32(h1);
+    };
+    if (ncand <= 64) sort(std::integral_constant<int, 1>{});
+    else if (ncand <= 128) sort(std::integral_constant<int, 2>{});
+    else if (ncand <= 256) sort(std::integral_constant<int, 4>{});
+    else sort(std::integral_constant<int, 8>{});
+  } else {
+    int npad = 1;
+    while (npad < ncand) npad <<= 1;
+    for (int c = ncand + lane; c < npad; c += 64) keys[c] = ~0ull;
+    wave_sync_lds();
+    for (int span = 2; span <= npad; span <<= 1) {
+      for (int j = span >> 1; j > 0; j >>= 1) {
+        for (int i = lane; i < npad; i += 64) {
+          const int p = i ^ j;
+          if (p > i) {
+            const uint64_t x = keys[i], y = keys[p];
+            if ((x > y) == ((i & span) == 0)) {
+              keys[i] = y;
+              keys[p] = x;
+            }
+          }
+        }
+        wave_sync_lds();
+      }
     }
+    for (int i = lane; i < nv; i += 64) put(i, (uint32_t)keys[i], ~(uint32_t)(keys[i] >> 32));
+    if (nv >= 1) top0 = key_to_f32(~(uint32_t)(keys[0] >> 32));
+    if (nv >= 2) top1 = key_to_f32(~(uint32_t)(keys[1] >> 32));
+  }
+  for (int i = kq + lane; i < kk; i += 64) {
+    oi[i] = 0;
+    os[i] = -FLT_MAX;
+    ov[i] = 0;
   }
   if (nv < kq) {
     const int need = kq - nv;
@@ -1045,8 +1080,8 @@ __global__ __launch_bounds__(64) void block_cand_kernel(BlockArgs a, float mscal
   }
   if (lane == 0) {
     a.counts[row] = kq;
-    a.top2[2 * row] = nv >= 1 ? key_to_f32(~(uint32_t)(keys[0] >> 32)) : -FLT_MAX;
-    a.top2[2 * row + 1] = nv >= 2 ? key_to_f32(~(uint32_t)(keys[1] >> 32)) : -FLT_MAX;
+    a.top2[2 * row] = top0;
+    a.top2[2 * row + 1] = top1;
   }
 }
 

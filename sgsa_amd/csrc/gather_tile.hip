@@ -598,7 +598,7 @@ __global__ __launch_bounds__(256, 2) void gather_thr_kernel(GatherArgs a, const 
   const int BH = a.B * a.H;
   const int bid = blockIdx.x;
   const int bh = bid % BH;
-  const int qb2 = nqb2 - 1 - bid / BH;   // heaviest row blocks first
+  const int qb2 = nqb2 - 1 - causal_block(bid / BH, nqb2, BH);
   const int b = bh / a.H, h = bh % a.H;
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform
   const int lr = lane & 15, lg = lane >> 4;
@@ -891,7 +891,7 @@ __global__ __launch_bounds__(256, 2) void dense_attn_kernel(DenseAttnArgs a, int
   const int BH = a.B * a.H;
   const int bid = blockIdx.x;
   const int bh = bid % BH;
-  const int qb2 = nqb2 - 1 - bid / BH;   // heaviest row blocks first
+  const int qb2 = nqb2 - 1 - causal_block(bid / BH, nqb2, BH);
   const int b = bh / a.H, h = bh % a.H, kh = h / (a.H / a.Hkv);
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, lg = lane >> 4;

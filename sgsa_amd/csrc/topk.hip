@@ -1750,7 +1750,7 @@ __global__ __launch_bounds__(256, 2) void score_thr128_kernel(TopkArgs a, int nq
   const int nqr = (a.Tq + QR - 1) / QR;
   const int bid = blockIdx.x;
   const int bh = bid % BH;
-  const int qb = nqr - 1 - bid / BH;   // heaviest (latest) row blocks first
+  const int qb = nqr - 1 - causal_block(bid / BH, nqr, BH);
   const int b = bh / a.H, h = bh % a.H;
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, lg = lane >> 4;

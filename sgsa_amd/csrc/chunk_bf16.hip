@@ -337,12 +337,18 @@ __global__ __launch_bounds__(64 * K3W) void chunk_inv_bf16(const bf16_t* __restr
 // K4: the state passes.
 // ---------------------------------------------------------------------------
 
-// Number of segments of the state pass: enough (b*h, segment) blocks to fill
-// the GPU, at least 8 chunks per segment, at most 16 segments.
+// Number of segments of the state pass: as many (b*h, segment) workgroups as one round of the
+// 256 CUs holds (one to a CU), segments of at least 4 chunks, at most 32 of them.  A workgroup alone
+// on its CU walks its chunks at the latency of each one, so shorter segments pay until the two
+// passes and the scan between them cost more than the chunks they save.  Whole forward, D = 128, with
+// segments of 8 chunks and half as many workgroups, then so: 16 heads T = 4096 241 -> 185 us, 2048
+// 212 -> 139, 1024 201 -> 121, 576 134 -> 95; one head T = 4096 210 -> 148; 200 heads T = 2048 (one
+// segment instead of two that do not fit in one round) 969 -> 551.  Eight chunks or fewer stay in one
+// segment: 16 heads T = 512 100 us, in two segments 112.
 inline int seg_count(int BH, int NT) {
-  int g = (256 + BH - 1) / BH;
-  g = g < 16 ? g : 16;
-  const int gmax = (NT + 7) / 8;
+  int g = 256 / BH;
+  g = g < 32 ? g : 32;
+  const int gmax = NT <= 8 ? 1 : (NT + 3) / 4;
   g = g < gmax ? g : gmax;
   return g < 1 ? 1 : g;
 }

@@ -117,21 +117,81 @@ __device__ __forceinline__ f4 f4_zero() {
 __device__ __forceinline__ int lane_id() { return threadIdx.x & 63; }
 __device__ __forceinline__ int wave_id() { return threadIdx.x >> 6; }
 
+// x of lane ^ M in VALU instructions: DPP within a row of 16 lanes, the row and half swaps across
+// rows.  A shuffle through LDS takes an address, a trip to LDS and a wait per
+// word: block retrieval's gather (131072 rows of 64 slots, some 20 reductions each) 214 us with those,
+// 204 so.
+template <int M>
+__device__ __forceinline__ uint32_t lane_xor(uint32_t x, int lane) {
+  const int v = (int)x;
+  if constexpr (M == 1) return (uint32_t)__builtin_amdgcn_update_dpp(0, v, 0xb1, 0xf, 0xf, true);         // quad_perm 1 0 3 2
+  else if constexpr (M == 2) return (uint32_t)__builtin_amdgcn_update_dpp(0, v, 0x4e, 0xf, 0xf, true);    // quad_perm 2 3 0 1
+  else if constexpr (M == 4) {   // lane ^ 7 (row_half_mirror), then ^ 3 (quad_perm 3 2 1 0)
+    const int y = __builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, true);
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, y, 0x1b, 0xf, 0xf, true);
+  } else if constexpr (M == 8) return (uint32_t)__builtin_amdgcn_update_dpp(0, v, 0x128, 0xf, 0xf, true);  // row_ror 8
+  else if constexpr (M == 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);   // even rows twice, odd rows twice
+    return (lane & 16) ? r[0] : r[1];
+  } else {
+    const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);   // low half twice, high half twice
+    return (lane & 32) ? r[0] : r[1];
+  }
+}
+__device__ __forceinline__ uint32_t lane_xor(uint32_t x, int m, int lane) {   // m a constant after unrolling
+  switch (m) {
+    case 1: return lane_xor<1>(x, lane);
+    case 2: return lane_xor<2>(x, lane);
+    case 4: return lane_xor<4>(x, lane);
+    case 8: return lane_xor<8>(x, lane);
+    case 16: return lane_xor<16>(x, lane);
+    default: return lane_xor<32>(x, lane);
+  }
+}
+
+// op(v, v of lane ^ o), op commutative: at 16 and 32 the two words of the swap are the pair.
+template <typename Op>
+__device__ __forceinline__ float xor_op(float v, int o, Op op) {
+  const uint32_t x = __float_as_uint(v);
+  if (o == 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  }
+  if (o == 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  }
+  return op(v, __uint_as_float(lane_xor(x, o, 0)));
+}
+__device__ __forceinline__ float xor_add(float v, int o) {
+  return xor_op(v, o, [](float a, float b) { return a + b; });
+}
+__device__ __forceinline__ float xor_max(float v, int o) {
+  return xor_op(v, o, [](float a, float b) { return fmaxf(a, b); });
+}
+
+__device__ __forceinline__ float xor_lane(float v, int o) {
+  return __uint_as_float(lane_xor(__float_as_uint(v), o, lane_id()));
+}
+
+// Whole waves only (every lane active), as the two below.
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  for (int o = 32; o > 0; o >>= 1) v = xor_add(v, o);
   return v;
 }
 
 __device__ __forceinline__ float wave_max(float v) {
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
+  for (int o = 32; o > 0; o >>= 1) v = xor_max(v, o);
   return v;
 }
 
-// Sum over the aligned group of `w` lanes containing this lane (w a power of 2, <= 64).
+// Sum over the aligned group of `w` lanes containing this lane (w a constant power of 2, <= 64).
 __device__ __forceinline__ float group_sum(float v, int w) {
-  for (int o = w >> 1; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1)
+    if (o < w) v = xor_add(v, o);
   return v;
 }
 

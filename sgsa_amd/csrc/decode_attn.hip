@@ -86,7 +86,7 @@ __global__ __launch_bounds__(256) void dattn_scores_kernel(const X* __restrict__
     if (valid) st(sws, ((long)b * H + kh * G + g) * kend + j, s[g]);
     m[g] = valid ? s[g] : -INFINITY;
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) m[g] = fmaxf(m[g], __shfl_xor(m[g], o, 64));
+    for (int o = 32; o > 0; o >>= 1) m[g] = xor_max(m[g], o);
     if (lane == 0) red[g][w][0] = m[g];
   }
   __syncthreads();
@@ -95,7 +95,7 @@ __global__ __launch_bounds__(256) void dattn_scores_kernel(const X* __restrict__
     m[g] = fmaxf(fmaxf(red[g][0][0], red[g][1][0]), fmaxf(red[g][2][0], red[g][3][0]));
     float e = valid ? expf(s[g] - m[g]) : 0.f;
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) e += __shfl_xor(e, o, 64);
+    for (int o = 32; o > 0; o >>= 1) e = xor_add(e, o);
     if (lane == 0) red[g][w][1] = e;
   }
   __syncthreads();
@@ -166,7 +166,7 @@ __global__ __launch_bounds__(256) void dattn_scores_mfma_kernel(const bf16_t* __
 #pragma unroll
   for (int e = 0; e < NE; ++e) {
 #pragma unroll
-    for (int o = 1; o < 16; o <<= 1) mh[e] = fmaxf(mh[e], __shfl_xor(mh[e], o, 64));
+    for (int o = 1; o < 16; o <<= 1) mh[e] = xor_max(mh[e], o);
     if (hl && lc == 0) red[4 * lg + e][w][0] = mh[e];
   }
   __syncthreads();
@@ -178,7 +178,7 @@ __global__ __launch_bounds__(256) void dattn_scores_mfma_kernel(const bf16_t* __
 #pragma unroll
     for (int kg = 0; kg < 4; ++kg) x += j0 + 16 * kg + lc < kend ? expf(sc[kg][e] - m) : 0.f;
 #pragma unroll
-    for (int o = 1; o < 16; o <<= 1) x += __shfl_xor(x, o, 64);
+    for (int o = 1; o < 16; o <<= 1) x = xor_add(x, o);
     if (hl && lc == 0) red[4 * lg + e][w][1] = x;
   }
   __syncthreads();
@@ -207,11 +207,11 @@ __global__ __launch_bounds__(256) void dattn_pv_kernel(const X* __restrict__ sws
     float mx = -INFINITY;
     for (int i = lane; i < nblk; i += 64) mx = fmaxf(mx, pp[i].x);
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    for (int o = 32; o > 0; o >>= 1) mx = xor_max(mx, o);
     float sum = 0.f;
     for (int i = lane; i < nblk; i += 64) sum += pp[i].y * expf(pp[i].x - mx);
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+    for (int o = 32; o > 0; o >>= 1) sum = xor_add(sum, o);
     if (lane == 0) { nm[w][0] = mx; nm[w][1] = sum; }
   }
   if (G > 4) {   // heads 4.. by the waves again
@@ -222,11 +222,11 @@ __global__ __launch_bounds__(256) void dattn_pv_kernel(const X* __restrict__ sws
       float mx = -INFINITY;
       for (int i = lane; i < nblk; i += 64) mx = fmaxf(mx, pp[i].x);
 #pragma unroll
-      for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+      for (int o = 32; o > 0; o >>= 1) mx = xor_max(mx, o);
       float sum = 0.f;
       for (int i = lane; i < nblk; i += 64) sum += pp[i].y * expf(pp[i].x - mx);
 #pragma unroll
-      for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+      for (int o = 32; o > 0; o >>= 1) sum = xor_add(sum, o);
       if (lane == 0) { nm[g][0] = mx; nm[g][1] = sum; }
     }
   }

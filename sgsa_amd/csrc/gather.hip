@@ -252,7 +252,7 @@ __device__ __forceinline__ void gather_slots_rescored(const GatherArgs& a, int s
         acc = fmaf(qv[2 * e + 1], __uint_as_float(wv[e] & 0xffff0000u), acc);
       }
 #pragma unroll
-      for (int o = 1; o < 16; o <<= 1) acc += __shfl_xor(acc, o, 64);
+      for (int o = 1; o < 16; o <<= 1) acc = xor_add(acc, o);
       const float sco = (okm >> u) & 1u ? acc * ms : 0.f;
       mine = sub == u ? sco : mine;
     }
@@ -289,6 +289,20 @@ __device__ __forceinline__ void gather_slots_rescored(const GatherArgs& a, int s
       unpack_row<bf16_t>(rk[u], xk);
 #pragma unroll
       for (int i = 0; i < 8; ++i) ak[i] += wv * xk[i];
+    }
+  }
+}
+
+// Sums ak and av over the wave's groups of lpr lanes (lanes with equal position in their group).
+template <int NE>
+__device__ __forceinline__ void sum_groups(float (&ak)[NE], float (&av)[NE], int lpr) {
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    if (o < lpr) continue;
+#pragma unroll
+    for (int i = 0; i < NE; ++i) {
+      ak[i] = xor_add(ak[i], o);
+      av[i] = xor_add(av[i], o);
     }
   }
 }
@@ -473,20 +487,14 @@ __device__ __forceinline__ void gather_row(const GatherArgs& a, long row, int lp
     }
   }
   // combine the groups (lanes with equal `sub`)
-  for (int o = lpr; o < 64; o <<= 1) {
-#pragma unroll
-    for (int i = 0; i < NE; ++i) {
-      ak[i] += __shfl_xor(ak[i], o, 64);
-      av[i] += __shfl_xor(av[i], o, 64);
-    }
-  }
+  sum_groups(ak, av, lpr);
   float s0 = mrun, s1;
   if (fixed_max) {
     s1 = a.top2[2 * row + 1];
   } else {
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
-      const float b1 = __shfl_xor(t1, o, 64), b2 = __shfl_xor(t2, o, 64);
+      const float b1 = xor_lane(t1, o), b2 = xor_lane(t2, o);
       const float hi = fmaxf(t1, b1), lo = fmaxf(fminf(t1, b1), fmaxf(t2, b2));
       t1 = hi; t2 = lo;
     }
@@ -573,11 +581,11 @@ __device__ __forceinline__ void gather_row(const GatherArgs& a, long row, int lp
 
   // ---- second pass over the slot list: weights, entropy, distance stats ----
   if (a.diag != nullptr || a.weights != nullptr) {
-    float ent = 0.f, dsum = 0.f, nloc = 0.f, nsink = 0.f, nrem = 0.f;
-    int imax = 0;
+    float ent = 0.f, dsum = 0.f;
+    int nloc = 0, nsink = 0, nrem = 0, imax = 0;   // the counts wave-uniform
     for (int base = 0; base < topk; base += 64) {
       const int slot = base + lane;
-      if (slot >= topk) break;
+      const bool in = slot < topk;
       int j = 0;
       float wv = 0.f;
       if (slot < kq) {
@@ -585,24 +593,23 @@ __device__ __forceinline__ void gather_row(const GatherArgs& a, long row, int lp
         const bool ok = vp ? (vp[slot] != 0) : true;
         wv = ok ? __expf(scp[slot] - mrun) * inv : 0.f;
       }
-      if (a.weights) a.weights[row * topk + slot] = wv;
+      if (a.weights && in) a.weights[row * topk + slot] = wv;
+      if (a.diag == nullptr) continue;
       const float wc = fmaxf(wv, eps);
-      ent += wc * logf(wc);
+      ent += in ? wc * logf(wc) : 0.f;
       const int dist = max(pos - j, 0);
-      dsum += (float)dist;
-      nloc += dist <= a.local_window ? 1.f : 0.f;
-      nsink += j < a.sink_size ? 1.f : 0.f;
-      nrem += (dist > a.local_window && j >= a.sink_size) ? 1.f : 0.f;
+      dsum += in ? (float)dist : 0.f;
+      const bool far = dist > a.local_window, sink = j < a.sink_size;
+      nloc += popc64(ballot64(in && !far));
+      nsink += popc64(ballot64(in && sink));
+      nrem += popc64(ballot64(in && far && !sink));
       imax = max(imax, j);
     }
     if (a.diag != nullptr) {
       ent = wave_sum(ent) + a.ent_pad * (eps * logf(eps));
       dsum = wave_sum(dsum);
-      nloc = wave_sum(nloc);
-      nsink = wave_sum(nsink);
-      nrem = wave_sum(nrem);
 #pragma unroll
-      for (int o = 32; o > 0; o >>= 1) imax = max(imax, __shfl_xor(imax, o, 64));
+      for (int o = 32; o > 0; o >>= 1) imax = max(imax, (int)lane_xor((uint32_t)imax, o, lane));
       if (lane == 0) {
         const long plane = (long)a.B * a.H * a.Tq;
         const float inv_k = 1.f / (float)topk;
@@ -614,9 +621,9 @@ __device__ __forceinline__ void gather_row(const GatherArgs& a, long row, int lp
         dg[4 * plane + row] = fminf(fmaxf(dot / (self_norm * kh_norm + eps), -1.f), 1.f);
         dg[5 * plane + row] = -ent;
         dg[6 * plane + row] = dsum * inv_k;    // divided by (max index + 1) in finish_diag
-        dg[7 * plane + row] = nloc * inv_k;
-        dg[8 * plane + row] = nsink * inv_k;
-        dg[9 * plane + row] = nrem * inv_k;
+        dg[7 * plane + row] = (float)nloc * inv_k;
+        dg[8 * plane + row] = (float)nsink * inv_k;
+        dg[9 * plane + row] = (float)nrem * inv_k;
         atomicMax(a.max_index + (row & (GATHER_MAXIDX_SLOTS - 1)), imax);   // spread: one word takes 1/64 of the rows
       }
     }
@@ -636,7 +643,7 @@ __global__ __launch_bounds__(256) void finish_diag_kernel(float* __restrict__ av
   if (threadIdx.x < 64) {
     int m = max_index[threadIdx.x & (GATHER_MAXIDX_SLOTS - 1)];
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o, 64));
+    for (int o = 32; o > 0; o >>= 1) m = max(m, (int)lane_xor((uint32_t)m, o, (int)threadIdx.x));
     if (threadIdx.x == 0) mx = m;
   }
   __syncthreads();
@@ -691,16 +698,10 @@ __global__ __launch_bounds__(256) void gather_part_kernel(GatherArgs a, int lpr)
                          reinterpret_cast<const X*>(a.v), b, h, grp, sub, lpr, fixed_max, mrun, t1, t2, esum, ak,
                          av);
   }
-  for (int o = lpr; o < 64; o <<= 1) {
-#pragma unroll
-    for (int i = 0; i < NE; ++i) {
-      ak[i] += __shfl_xor(ak[i], o, 64);
-      av[i] += __shfl_xor(av[i], o, 64);
-    }
-  }
+  sum_groups(ak, av, lpr);
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
-    const float b1 = __shfl_xor(t1, o, 64), b2 = __shfl_xor(t2, o, 64);
+    const float b1 = xor_lane(t1, o), b2 = xor_lane(t2, o);
     const float hi = fmaxf(t1, b1), lo = fmaxf(fminf(t1, b1), fmaxf(t2, b2));
     t1 = hi; t2 = lo;
   }
@@ -867,7 +868,7 @@ __global__ __launch_bounds__(256) void rescore_kernel(int B, int Tq, int Tk, int
           acc = fmaf(qv[2 * e + 1], __uint_as_float(wv[e] & 0xffff0000u), acc);
         }
 #pragma unroll
-        for (int o = 1; o < 16; o <<= 1) acc += __shfl_xor(acc, o, 64);
+        for (int o = 1; o < 16; o <<= 1) acc = xor_add(acc, o);
         const int i = base + 4 * u + grp;
         if (i < nend && l16 == 0) sp[i] = ok[u] ? acc * mscale : 0.f;
       }
@@ -888,7 +889,7 @@ __global__ __launch_bounds__(256) void rescore_kernel(int B, int Tq, int Tk, int
       }
     }
 #pragma unroll
-    for (int o = 1; o < 16; o <<= 1) acc += __shfl_xor(acc, o, 64);
+    for (int o = 1; o < 16; o <<= 1) acc = xor_add(acc, o);
     if (i < nend && l16 == 0) sp[i] = acc * mscale;
   }
 }

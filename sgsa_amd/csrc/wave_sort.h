@@ -7,36 +7,6 @@
 
 namespace sgsa {
 
-// x of lane ^ M in VALU instructions: DPP within a row of 16 lanes, the row and half swaps across
-// rows (a shuffle through LDS takes an address and a wait per word).
-template <int M>
-__device__ __forceinline__ uint32_t lane_xor(uint32_t x, int lane) {
-  const int v = (int)x;
-  if constexpr (M == 1) return (uint32_t)__builtin_amdgcn_update_dpp(v, v, 0xb1, 0xf, 0xf, false);         // quad_perm 1 0 3 2
-  else if constexpr (M == 2) return (uint32_t)__builtin_amdgcn_update_dpp(v, v, 0x4e, 0xf, 0xf, false);    // quad_perm 2 3 0 1
-  else if constexpr (M == 4) {   // lane ^ 7 (row_half_mirror), then ^ 3 (quad_perm 3 2 1 0)
-    const int y = __builtin_amdgcn_update_dpp(v, v, 0x141, 0xf, 0xf, false);
-    return (uint32_t)__builtin_amdgcn_update_dpp(y, y, 0x1b, 0xf, 0xf, false);
-  } else if constexpr (M == 8) return (uint32_t)__builtin_amdgcn_update_dpp(v, v, 0x128, 0xf, 0xf, false);  // row_ror 8
-  else if constexpr (M == 16) {
-    const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);   // even rows twice, odd rows twice
-    return (lane & 16) ? r[0] : r[1];
-  } else {
-    const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);   // low half twice, high half twice
-    return (lane & 32) ? r[0] : r[1];
-  }
-}
-__device__ __forceinline__ uint32_t lane_xor(uint32_t x, int m, int lane) {   // m a constant after unrolling
-  switch (m) {
-    case 1: return lane_xor<1>(x, lane);
-    case 2: return lane_xor<2>(x, lane);
-    case 4: return lane_xor<4>(x, lane);
-    case 8: return lane_xor<8>(x, lane);
-    case 16: return lane_xor<16>(x, lane);
-    default: return lane_xor<32>(x, lane);
-  }
-}
-
 template <int NS>
 __device__ __forceinline__ void wave_sort_desc(uint32_t (&hi)[NS], uint32_t (&lo)[NS], int lane) {
   // x is kept where it is the larger (max) or smaller of the pair

@@ -203,6 +203,133 @@ __device__ __forceinline__ void gather_slots(const GatherArgs& a, int s0, int s1
   }
 }
 
+// The weighted sums of bf16 rows on the matrix cores (sums of one query row: nothing is shared between
+// query rows, so the product is v_mfma_f32_4x4x4_16b_bf16, one 4x4 block to four lanes).  A lane holds
+// the same 8 dims of four slots' rows; eight products take a dim each: B[k][lane % 4] the lane's element
+// of slot k, A[i][k] part i of slot k's weight.  An fp32 weight is the exact sum of three bf16 parts (8
+// bits of mantissa each), the rows of A, so every product is exact and the four terms are summed in
+// fp32 as before.  Per four slots and 8 dims that is 16 permutes and 8 products where unpacking and
+// fused multiply-adds took 64 instructions, which bound the plain form.  65536 rows of D = 128 and 256
+// slots: value rows 295 -> 183 us, key and value rows 413 -> 318; 64 slots 120 -> 81 and 158 -> 122; what
+// bounds it now is the rows' delivery from L2 (8.6 GB at 27 TB/s with both).  Four or five waves to a
+// SIMD (launch bounds) before more loads in flight in each: eight slots a step without key rows 206.
+// A lane group of LPR lanes (LPR >= 4, a multiple of the block) takes four consecutive slots a step;
+// the slots' row offsets and weight parts pass through LDS, one write per slot and one read per step.
+// A part of 0 times an inf is a NaN that the plain product does not have: the caller takes the plain
+// form for a row whose sums are not finite.
+struct GatherLds {
+  uint32_t off[64];        // byte offset of the slot's row from the (b, h) base
+  uint16_t part[4][64];    // the weight's leading, next and last 8 bits; zeros
+};
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+
+// One step's four rows into the sums.
+__device__ __forceinline__ void mx_add(const uint4 (&r)[4], s16x4 pw, f4 (&acc)[8]) {
+  const uint32_t x[4][4] = {{r[0].x, r[0].y, r[0].z, r[0].w}, {r[1].x, r[1].y, r[1].z, r[1].w},
+                            {r[2].x, r[2].y, r[2].z, r[2].w}, {r[3].x, r[3].y, r[3].z, r[3].w}};
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const uint32_t sel = e ? 0x07060302u : 0x05040100u;
+      const uint2 y = make_uint2(__builtin_amdgcn_perm(x[1][q], x[0][q], sel),
+                                 __builtin_amdgcn_perm(x[3][q], x[2][q], sel));
+      acc[2 * q + e] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(pw, __builtin_bit_cast(s16x4, y), acc[2 * q + e], 0, 0, 0);
+    }
+}
+
+// gather_slots of all kq slots of a row in that form (KP: key rows too); false where a sum is not finite.
+template <bool KP>
+__device__ __forceinline__ bool gather_slots_mx(const GatherArgs& a, int kq, const int32_t* idxp, const float* scp,
+                                                const uint8_t* vp, const char* K, const char* V, int grp, int sub,
+                                                int lpr, bool fixed_max, float& mrun, float& t1, float& t2,
+                                                float& esum, float (&ak)[8], float (&av)[8], GatherLds& L) {
+  const int lane = threadIdx.x & 63;
+  const uint32_t stride = (uint32_t)(a.kv_hm ? a.D : a.H * a.D) * 2u;
+  const uint32_t dim = sub * 8 < a.D ? 16u * (uint32_t)sub : 0u;
+  const int rpi = 64 / lpr;
+  f4 sk[KP ? 8 : 1], sv[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    if constexpr (KP) sk[i] = f4_zero();
+    sv[i] = f4_zero();
+  }
+  L.part[3][lane] = 0;
+  // the next 64 slots are loaded under the current ones' rows
+  int jn = 0;
+  float sn = -INFINITY;
+  auto load = [&](int slot) {
+    jn = 0;
+    sn = -INFINITY;
+    if (slot < kq) {
+      jn = idxp[slot];
+      if (vp == nullptr || vp[slot] != 0) sn = scp[slot];
+    }
+  };
+  load(lane);
+  for (int base = 0; base < kq; base += 64) {
+    const int j = jn;
+    const float sc = sn;
+    load(base + 64 + lane);
+    if (!fixed_max) {
+      const float bm = wave_max(sc);
+      if (bm > mrun) {
+        const float f = (mrun == -INFINITY) ? 0.f : __expf(mrun - bm);
+        esum *= f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          if constexpr (KP) sk[i] *= f;
+          sv[i] *= f;
+        }
+        mrun = bm;
+      }
+      const float so = sc == -INFINITY ? -FLT_MAX : sc;
+      t2 = fmaxf(t2, fminf(t1, so));
+      t1 = fmaxf(t1, so);
+    }
+    const float wgt = sc == -INFINITY ? 0.f : __expf(sc - mrun);
+    esum += wgt;
+    const float w1 = wgt - __uint_as_float(__float_as_uint(wgt) & 0xffff0000u);
+    const float w2 = w1 - __uint_as_float(__float_as_uint(w1) & 0xffff0000u);
+    __builtin_amdgcn_wave_barrier();   // the last block's reads come first (one wave's LDS accesses stay in order)
+    L.off[lane] = (uint32_t)j * stride;
+    L.part[0][lane] = (uint16_t)(__float_as_uint(wgt) >> 16);
+    L.part[1][lane] = (uint16_t)(__float_as_uint(w1) >> 16);
+    L.part[2][lane] = (uint16_t)(__float_as_uint(w2) >> 16);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const int nstep = min(64, kq - base);
+#pragma unroll 1
+    for (int it = 0; it * rpi * 4 < nstep; ++it) {
+      const int s4 = 4 * (it * rpi + grp);
+      const uint4 o = *reinterpret_cast<const uint4*>(&L.off[s4]);
+      const s16x4 pw = *reinterpret_cast<const s16x4*>(&L.part[lane & 3][s4]);
+      const uint32_t off[4] = {o.x + dim, o.y + dim, o.z + dim, o.w + dim};
+      uint4 rv[4], rk[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        rv[u] = *reinterpret_cast<const uint4*>(V + off[u]);
+        if constexpr (KP) rk[u] = *reinterpret_cast<const uint4*>(K + off[u]);
+      }
+      __builtin_amdgcn_sched_barrier(0);   // every load issued before a product waits for the first
+      mx_add(rv, pw, sv);
+      if constexpr (KP) mx_add(rk, pw, sk);
+    }
+  }
+  bool ok = true;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    av[i] = sub * 8 < a.D ? sv[i][0] + (sv[i][1] + sv[i][2]) : 0.f;
+    ok = ok && fabsf(av[i]) < INFINITY;
+    if constexpr (KP) {
+      ak[i] = sub * 8 < a.D ? sk[i][0] + (sk[i][1] + sk[i][2]) : 0.f;
+      ok = ok && fabsf(ak[i]) < INFINITY;
+    }
+  }
+  return ballot64(!ok) == 0;
+}
+
 // gather_slots for bf16 rows of D = 128 ([B,Tk,H,D], 16 lanes per row) whose slot scores
 // are computed here, from the query's 8 elements of the lane (qv) and the key rows the
 // gather loads anyway: each 64-slot block loads its 64 key and value rows (lane group g:
@@ -311,12 +438,14 @@ __device__ __forceinline__ void sum_groups(float (&ak)[NE], float (&av)[NE], int
 // epilogue.  Wave-local: no LDS and no block barrier.
 // PA: the split partials are 16-byte aligned (the launcher checks a.part), so their row pieces
 // load 16 bytes at a time.
-template <typename X, bool VEC, bool SPLIT, bool PA = false>
-__device__ __forceinline__ void gather_row(const GatherArgs& a, long row, int lpr) {
+// Returns the largest key index of the row's slots with diagnostics, else 0.
+// MX: the sums on the matrix cores, without (1) or with (2) key rows, by way of lds.
+template <typename X, bool VEC, bool SPLIT, bool PA = false, int MX = 0>
+__device__ __forceinline__ int gather_row(const GatherArgs& a, long row, int lpr, GatherLds* lds = nullptr) {
   constexpr int NE = GatherShape<X, VEC>::NE;
   const int lane = threadIdx.x & 63;
   const long nrows = (long)a.B * a.H * a.Tq;
-  if (row >= nrows) return;
+  if (row >= nrows) return 0;
   const int Tq = a.Tq, H = a.H, D = a.D, topk = a.top_k;
   const int bh = (int)(row / Tq), qr = (int)(row % Tq);
   const int b = bh / H, h = bh % H;
@@ -337,46 +466,37 @@ __device__ __forceinline__ void gather_row(const GatherArgs& a, long row, int lp
 #pragma unroll
   for (int i = 0; i < NE; ++i) { ak[i] = 0.f; av[i] = 0.f; }
   float esum = 0.f;
-  // the epilogue's own inputs, loaded first (they do not depend on the slots)
+  // the epilogue's own inputs, loaded first (they do not depend on the slots; last where registers are short)
   const long qoff = ((long)(b * Tq + qr) * H + h) * D;
   float kt[NE];
-  if (a.self_key != nullptr && (a.diag != nullptr || a.budget != nullptr)) {
-    load_row<X, VEC>(reinterpret_cast<const X*>(a.self_key), qoff, sub, D, lpr, kt);
-  } else {
+  auto load_self = [&]() {
+    if (a.self_key != nullptr && (a.diag != nullptr || a.budget != nullptr)) {
+      load_row<X, VEC>(reinterpret_cast<const X*>(a.self_key), qoff, sub, D, lpr, kt);
+    } else {
 #pragma unroll
-    for (int i = 0; i < NE; ++i) kt[i] = 0.f;
-  }
+      for (int i = 0; i < NE; ++i) kt[i] = 0.f;
+    }
+  };
+  if constexpr (MX != 2) load_self();
   const float bud = a.budget != nullptr ? a.budget[(long)(b * Tq + qr) * H + h] : 0.f;
 
   if constexpr (!SPLIT) {
-    for (int base = 0; base < kq; base += 64) {
-      const int slot = base + lane;
-      int j = 0;
-      float sc = -INFINITY;
-      if (slot < kq) {
-        j = idxp[slot];
-        const bool ok = vp ? (vp[slot] != 0) : true;
-        if (ok) sc = scp[slot];
+    bool done = false;
+    if constexpr (MX > 0) {
+      const long hb = kv_row_offset(a, b, h, 0);
+      done = gather_slots_mx<MX == 2>(a, kq, idxp, scp, vp, reinterpret_cast<const char*>(K + hb),
+                                      reinterpret_cast<const char*>(V + hb), grp, sub, lpr, fixed_max, mrun, t1, t2,
+                                      esum, ak, av, *lds);
+      if (!done) {
+        if (!fixed_max) mrun = -INFINITY;
+        t1 = t2 = -FLT_MAX;
+        esum = 0.f;
+#pragma unroll
+        for (int i = 0; i < NE; ++i) { ak[i] = 0.f; av[i] = 0.f; }
       }
-      if (!fixed_max) {
-        // online-softmax merge: rescale what was accumulated under the old max
-        const float bm = wave_max(sc);
-        if (bm > mrun) {
-          const float f = (mrun == -INFINITY) ? 0.f : __expf(mrun - bm);
-          esum *= f;
-  #pragma unroll
-          for (int i = 0; i < NE; ++i) { ak[i] *= f; av[i] *= f; }
-          mrun = bm;
-        }
-        const float so = sc == -INFINITY ? -FLT_MAX : sc;
-        t2 = fmaxf(t2, fminf(t1, so));
-        t1 = fmaxf(t1, so);
-      }
-      const float wgt = sc == -INFINITY ? 0.f : __expf(sc - mrun);
-      esum += wgt;
-      const int nstep = min(64, kq - base);
-      gather_step<X, VEC>(a, j, wgt, nstep, K, V, b, h, grp, sub, lpr, ak, av);
     }
+    if (!done)
+      gather_slots<X, VEC>(a, 0, kq, idxp, scp, vp, K, V, b, h, grp, sub, lpr, fixed_max, mrun, t1, t2, esum, ak, av);
   } else {
     // merge the row's partials (gather_part_kernel): lane c takes partials c, c + 64, .. for the
     // sums and top-2 pairs; lane group g adds partials g, g + 64 / lpr, .. to the row vectors
@@ -486,6 +606,7 @@ __device__ __forceinline__ void gather_row(const GatherArgs& a, long row, int lp
     }
     }
   }
+  if constexpr (MX == 2) load_self();
   // combine the groups (lanes with equal `sub`)
   sum_groups(ak, av, lpr);
   float s0 = mrun, s1;
@@ -580,9 +701,10 @@ __device__ __forceinline__ void gather_row(const GatherArgs& a, long row, int lp
   if (a.alpha && lane == 0) a.alpha[(long)(b * Tq + qr) * H + h] = alpha_v;
 
   // ---- second pass over the slot list: weights, entropy, distance stats ----
+  int imax = 0;
   if (a.diag != nullptr || a.weights != nullptr) {
     float ent = 0.f, dsum = 0.f;
-    int nloc = 0, nsink = 0, nrem = 0, imax = 0;   // the counts wave-uniform
+    int nloc = 0, nsink = 0, nrem = 0;   // wave-uniform
     for (int base = 0; base < topk; base += 64) {
       const int slot = base + lane;
       const bool in = slot < topk;
@@ -624,15 +746,34 @@ __device__ __forceinline__ void gather_row(const GatherArgs& a, long row, int lp
         dg[7 * plane + row] = (float)nloc * inv_k;
         dg[8 * plane + row] = (float)nsink * inv_k;
         dg[9 * plane + row] = (float)nrem * inv_k;
-        atomicMax(a.max_index + (row & (GATHER_MAXIDX_SLOTS - 1)), imax);   // spread: one word takes 1/64 of the rows
       }
     }
   }
+  return imax;
+}
+
+// One atomic for the block's four rows, spread over the words: an atomic to the words' two cache lines
+// takes 3.5 ns, so one for every row bounded the diagnostics (65536 rows of 8 slots: 323 us against 96
+// without diagnostics; now 134 against 88).
+__device__ __forceinline__ void block_max_index(const GatherArgs& a, int imax) {
+  __shared__ int m[4];
+  if (a.diag == nullptr) return;
+  if ((threadIdx.x & 63) == 0) m[threadIdx.x >> 6] = imax;
+  __syncthreads();
+  if (threadIdx.x == 0)
+    atomicMax(a.max_index + (blockIdx.x & (GATHER_MAXIDX_SLOTS - 1)), max(max(m[0], m[1]), max(m[2], m[3])));
 }
 
 template <typename X, bool VEC, bool SPLIT, bool PA = false>
 __global__ __launch_bounds__(256) void sparse_gather_kernel(GatherArgs a, int lpr) {
-  gather_row<X, VEC, SPLIT, PA>(a, (long)blockIdx.x * 4 + (threadIdx.x >> 6), lpr);
+  block_max_index(a, gather_row<X, VEC, SPLIT, PA>(a, (long)blockIdx.x * 4 + (threadIdx.x >> 6), lpr));
+}
+
+template <bool KP>
+__global__ __launch_bounds__(256, KP ? 4 : 5) void sparse_gather_mx_kernel(GatherArgs a, int lpr) {
+  __shared__ __align__(16) GatherLds lds[4];
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  block_max_index(a, gather_row<bf16_t, true, false, false, KP ? 2 : 1>(a, (long)blockIdx.x * 4 + w, lpr, &lds[w]));
 }
 
 // avg_distance /= max(max_index + 1, 1)  (modelings/modeling_sgsa.py:395, :401); the largest index is the
@@ -788,8 +929,12 @@ hipError_t launch_sparse_gather(const GatherArgs& a, hipStream_t st) {
       else if (sp) sparse_gather_kernel<float, true, true><<<grid, 256, 0, st>>>(a, lpr);
       else sparse_gather_kernel<float, true, false><<<grid, 256, 0, st>>>(a, lpr);
     } else {
+      // the matrix form needs four-lane blocks inside a lane group and a head's rows in 32 bits of bytes
+      const bool mx = lpr >= 4 && 2L * a.Tk * a.D * (a.kv_hm ? 1 : a.H) <= 0xffffffffL;
       if (pa) sparse_gather_kernel<bf16_t, true, true, true><<<grid, 256, 0, st>>>(a, lpr);
       else if (sp) sparse_gather_kernel<bf16_t, true, true><<<grid, 256, 0, st>>>(a, lpr);
+      else if (mx && a.k != nullptr) sparse_gather_mx_kernel<true><<<grid, 256, 0, st>>>(a, lpr);
+      else if (mx) sparse_gather_mx_kernel<false><<<grid, 256, 0, st>>>(a, lpr);
       else sparse_gather_kernel<bf16_t, true, false><<<grid, 256, 0, st>>>(a, lpr);
     }
   } else {

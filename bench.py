@@ -575,11 +575,11 @@ def run_backward(args) -> int:
     log(f"native backward ms/call {ms:.3f}")
     # fp32 MFMA multiply-adds per chunk-head (M = 2L samples with the sparse write, L tokens, d dims)
     M, L, d = 128, 64, 128
-    mac = (3 * M * M * d + M ** 3 // 3                                    # intra: Gram, (I+T)^-1, W, U
-           + 2 * d * d * M                                               # maps: Phi, Pm
+    mac = (M * M * d + M ** 3 // 3                                       # intra: Gram, (I+T)^-1
+           + M * M * d + 2 * d * d * M                                   # maps: A^T kappa, Phi, Pm
            + 2 * d ** 3                                                  # the two scans, one step each
-           + L * M * d + d * d * L + M * d * L + d * d * M               # pre: P, Q^T dO, P^T dO, W^T X1
-           + 5 * M * d * d + 7 * M * M * d + 2 * M ** 3 + 4 * L * M * d + L * d * d)   # gradient kernel
+           + L * M * d + d * d * L + M * d * L + M * M * d + d * d * M   # pre: P, Q^T dO, P^T dO, A^T X1, kappa^T
+           + 17_500_000)                                                 # gradient kernel (triangles cut at the tile)
     nchunks = B * H * ((T + 63) // 64)
     flops = 2.0 * mac * nchunks
     torch_ms = None

@@ -302,8 +302,8 @@ __global__ __launch_bounds__(4 * M) void chunk_maps_kernel(ChunkArgs f, const fl
 // A step is latency: 32 dependent MFMAs at DP = 128 and a barrier, about 2.9 us.  That is less
 // than a quarter of a step with a head's whole state in one workgroup (12 us), which is why the
 // chunks are not also split into segments: at B=4 T=4096 H=8 D=128 (64 chunks) 197 us against
-// 340 us for a segmented scan in three passes, at T = 32768 with 16 heads (512 chunks) 512 such
-// steps against 112 of the segmented form's, still the shorter.
+// 340 us for a segmented scan in three passes, and about even at T = 32768 with 16 heads, by
+// the steps' times (512 of these, 112 of the segmented form's).
 // ---------------------------------------------------------------------------
 template <int DP, bool TR>
 __global__ __launch_bounds__(4 * DP) void chunk_scan_kernel(const float* __restrict__ phi, const float* __restrict__ y,

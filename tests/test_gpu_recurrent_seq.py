@@ -38,3 +38,27 @@ def test_tokens_equal_single_steps(dev, dt, B, T, H, D, sparse, shift):
                                      output_final_state=True)
         assert torch.equal(o[:, t:t + 1], one), t
     assert torch.equal(end, st)
+
+
+@pytest.mark.parametrize("T,D,sparse", [(4, 128, True), (9, 128, False), (13, 64, True), (15, 65, True), (16, 128, True)])
+def test_infinite_last_write(dev, T, D, sparse):
+    """An infinite value written by the last token stays where it was written: the final state is that of
+    one-token calls, infinite entries and finite neighbours, whatever T leaves of the last chunk of 8."""
+    g = torch.Generator().manual_seed(43)
+    r = lambda *s: torch.randn(*s, generator=g)
+    unit = lambda t: t / t.norm(dim=-1, keepdim=True)
+    B, H = 2, 3
+    x = [unit(r(B, T, H, D)), unit(r(B, T, H, D)), r(B, T, H, D), torch.sigmoid(r(B, T, H)), torch.sigmoid(r(B, T, H) + 3.0)]
+    x += [unit(r(B, T, H, D)), r(B, T, H, D), 0.25 * torch.sigmoid(r(B, T, H))] if sparse else [None] * 3
+    x[2][0, -1, 1, 5] = float("inf")
+    x[1][0, -1, 1, 3] = 0.0   # inf * 0 in one row of that column
+    x = [None if t is None else t.to(dev) for t in x]
+    st = (0.1 * r(B, H, D, D)).to(dev)
+    print(f"recurrent seq infinite T={T} D={D} sparse={sparse}", flush=True)
+    o, end = recurrent_sgsa_fwd(*x, initial_state=st, output_final_state=True)
+    for t in range(T):
+        one, st = recurrent_sgsa_fwd(*(None if a is None else a[:, t:t + 1] for a in x), initial_state=st,
+                                     output_final_state=True)
+        assert torch.equal(o[:, t:t + 1].isnan(), one.isnan()) and torch.equal(o[:, t:t + 1].nan_to_num(), one.nan_to_num()), t
+    assert end[0, 1, :, 5].isinf().sum() == D - 1
+    assert torch.equal(end.isnan(), st.isnan()) and torch.equal(end.nan_to_num(), st.nan_to_num())

@@ -210,8 +210,10 @@ __global__ __launch_bounds__(64 * (M / 16)) void chunk_bwd_grad_kernel(ChunkBwdA
   constexpr int NTQ = NQ < 4 ? NQ : 4, NDQ = NQ / NTQ;
   __shared__ __align__(16) float P[PS0 > PS1 ? PS0 : PS1];   // S, then R, then the tiles of X and Y
   __shared__ __align__(16) float Q[(DP > M ? DP : M) * PD];  // B, then G, then dR, then kappa
-  __shared__ float lam[M], dlam[M];
-  __shared__ float logd[L], el[L], dl[L];
+  __shared__ float lam[M], logd[L], el[L];
+  // each wave's own part of dlambda and dl, added up in wave order at the end: the gate gradients repeat bit for
+  // bit, which atomics on one array shared by the waves did not
+  __shared__ __align__(16) float dlam[NW][M], dl[NW][L];
   __shared__ float red[NW];
   auto yidx = [](int I, int J) { return NTL + IPT * (I * (I + 1) / 2) + J; };
 
@@ -242,12 +244,11 @@ __global__ __launch_bounds__(64 * (M / 16)) void chunk_bwd_grad_kernel(ChunkBwdA
     const float x = lgd[cb * L + tid];
     logd[tid] = x;
     el[tid] = expf(x);
-    dl[tid] = 0.f;
   }
-  if (tid < M) {
-    lam[tid] = strength<M>(a.f, b, h, t0, tid);
-    dlam[tid] = 0.f;
-  }
+  if (tid < M) lam[tid] = strength<M>(a.f, b, h, t0, tid);
+  dl[w][lane] = 0.f;
+#pragma unroll
+  for (int u = 0; u < M / 64; ++u) dlam[w][64 * u + lane] = 0.f;
   __syncthreads();
   const float lami = lam[i], dec = expf(logd[L - 1] - logd[ti]), ci = lami * dec, ei = el[ti];
   float own_dlam = 0.f, own_dl = 0.f;   // this lane's part of sample i's dlambda and dl_tau
@@ -317,13 +318,14 @@ __global__ __launch_bounds__(64 * (M / 16)) void chunk_bwd_grad_kernel(ChunkBwdA
     }
 #pragma unroll
     for (int I = 0; I < NTQ; ++I) {
+      const int t = 16 * (tq0 + I) + 4 * lg;
+      f4 p;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {   // dl_t += e^l_t q_t . (S dO_t)
-        const int t = 16 * (tq0 + I) + 4 * lg + e;
-        dq[u][I][e] *= el[t];
-        const float p = sum_lr(q.uat(t, 16 * (dq0 + u) + lr) * dq[u][I][e]);
-        if (lr == 0) atomicAdd(&dl[t], p);
+        dq[u][I][e] *= el[t + e];
+        p[e] = sum_lr(q.uat(t + e, 16 * (dq0 + u) + lr) * dq[u][I][e]);
       }
+      if (lr == 0) *reinterpret_cast<f4*>(&dl[w][t]) += p;
     }
   }
   // <G, S>, for dl_L
@@ -386,24 +388,33 @@ __global__ __launch_bounds__(64 * (M / 16)) void chunk_bwd_grad_kernel(ChunkBwdA
     }
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      f4 xl;
+      const int j0 = 16 * (J0 + u) + 4 * lg;
+      f4 xl, s, sl;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int j = 16 * (J0 + u) + 4 * lg + e, tj = samp_t<M>(j);
+        const int j = j0 + e, tj = samp_t<M>(j);
         const float x = tj < ti ? -dt[u][e] * expf(logd[ti] - logd[tj]) : 0.f;
         const float xg = x * gk[u][e], lj = lam[j];
         xr[J0 + u][e] = x;
         xl[e] = x * lj;
         own_dl += xg * lj;
-        const float s = sum_lr(xg);
-        if (lr == 0) {
-          atomicAdd(&dlam[j], s);
-          atomicAdd(&dl[tj], -s * lj);
+        s[e] = sum_lr(xg);
+        sl[e] = s[e] * lj;
+      }
+      if (lr == 0) {
+        *reinterpret_cast<f4*>(&dlam[w][j0]) = s;   // the wave's only term for these samples
+        float* d = &dl[w][samp_t<M>(j0)];
+        if constexpr (SP) {
+          d[0] -= sl[0] + sl[1];
+          d[1] -= sl[2] + sl[3];
+        } else {
+          *reinterpret_cast<f4*>(d) -= sl;
         }
       }
       if (J0 + u <= it) mm_col<RT, PD>(dk, Q + (16 * (J0 + u) + 4 * lg) * PD + lr, xl);
     }
   }
+  wave_lds_sync();   // dl[w]: another lane's words from here on
   // Y and the P-terms of dlambda and dl; dkappa += Y^T Q
   f4 y[L / 16];
 #pragma unroll
@@ -419,6 +430,7 @@ __global__ __launch_bounds__(64 * (M / 16)) void chunk_bwd_grad_kernel(ChunkBwdA
         dp = mma_f32(x2[e], rr[n][e], dp);
       }
     }
+    f4 s;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int t = 16 * I + 4 * lg + e;
@@ -428,9 +440,9 @@ __global__ __launch_bounds__(64 * (M / 16)) void chunk_bwd_grad_kernel(ChunkBwdA
       own_dlam += de * qk[e];
       const float v = y[I][e] * qk[e];
       own_dl -= v;
-      const float s = sum_lr(v);
-      if (lr == 0) atomicAdd(&dl[t], s);
+      s[e] = sum_lr(v);
     }
+    if (lr == 0) *reinterpret_cast<f4*>(&dl[w][16 * I + 4 * lg]) += s;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       float x[RT];
@@ -494,14 +506,17 @@ __global__ __launch_bounds__(64 * (M / 16)) void chunk_bwd_grad_kernel(ChunkBwdA
   }
   own_dlam = sum_lg(own_dlam);
   own_dl = sum_lg(own_dl);
+  if constexpr (SP) own_dl = xor_add(own_dl, 1);   // a token's two samples are lanes 2n and 2n + 1
   if (lg == 0) {
-    atomicAdd(&dlam[i], own_dlam);
-    atomicAdd(&dl[ti], own_dl);
+    dlam[w][i] += own_dlam;
+    if (!SP || (lr & 1) == 0) dl[w][ti] += own_dl;
   }
   __syncthreads();
   // dgamma from the suffix sums of dl (one token per lane); dbeta / dalpha from dlambda
   if (w == 0) {
-    float x = dl[lane];
+    float x = 0.f;
+#pragma unroll
+    for (int u = 0; u < NW; ++u) x += dl[u][lane];
     if (lane == L - 1) {
 #pragma unroll
       for (int u = 0; u < NW; ++u) x += red[u];
@@ -522,8 +537,11 @@ __global__ __launch_bounds__(64 * (M / 16)) void chunk_bwd_grad_kernel(ChunkBwdA
     const int t = t0 + samp_t<M>(tid);
     if (t < T) {
       const long o = (long)(b * T + t) * H + h;
-      if (samp_r<M>(tid)) a.dalpha[o] = dlam[tid];
-      else a.dbeta[o] = dlam[tid];
+      float x = 0.f;
+#pragma unroll
+      for (int u = 0; u < NW; ++u) x += dlam[u][tid];
+      if (samp_r<M>(tid)) a.dalpha[o] = x;
+      else a.dbeta[o] = x;
     }
   }
 }

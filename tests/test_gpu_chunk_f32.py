@@ -58,3 +58,17 @@ def test_chunk_f32_edges(dev, dt, T, D, sparse, shift):
         assert torch.isfinite(a).all(), f"{name}: non-finite"
         err = ((a - b).abs().max() / b.abs().max().clamp_min(1e-12)).item()
         assert err <= tol, f"{name}: {err:.3e}"
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,D,sparse", [(1000, 128, True), (1000, 64, True), (700, 128, False), (700, 50, False)])
+def test_gradients_repeat(dev, dt, T, D, sparse):
+    """Fixed inputs give the same gradients bit for bit, the gates' (sums over a chunk's waves) among them."""
+    x, do, dht = _inputs(2, T, 6, D, dt, sparse, 0, dev)
+    print(f"gradients repeat {dt} T={T} D={D} sparse={sparse}", flush=True)
+    needs = [t is not None for t in x]
+    first = sgsa_amd.chunk_sgsa_bwd(x, needs, do, dht)
+    for _ in range(12):
+        again = sgsa_amd.chunk_sgsa_bwd(x, needs, do, dht)
+        for name, a, b in zip(NAMES, first, again):
+            assert a is None or torch.equal(a, b), name

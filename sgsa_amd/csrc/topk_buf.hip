@@ -24,7 +24,8 @@
 // heads 3013 -> 3132 unsorted, 3749 -> 3228 sorted); T=8192 1535 -> 2263, 2184 -> 2437.  D=64
 // T=4096 1189 -> 385, T=8192 k=512 5172 -> 2113.  fp32 D=64 T=2048 707 -> 191, D=128 T=8192 3557 ->
 // 3958.  So with D = 128, where the row kernel reads whole vectors, the line lies at 2048 keys, or
-// 4096 where this form also sorts; elsewhere at 8192, the registers' limit.
+// 4096 where this form also sorts; elsewhere at 8192, the registers' limit.  Unsorted rows that keep
+// most of their keys stay on the row kernel there (mostly_kept).
 //
 // Output contract as the row kernel: counts = min(slots, valid keys), slots past
 // it index 0 and -FLT_MAX, top2 the two largest valid scores, ties at the cut to
@@ -500,11 +501,30 @@ int buf_pitch(const TopkArgs& t) { return (t.Tk + KB - 1) / KB * KB + 64; }
 // Row blocks whose buffer rows fit the row kernel's candidate lists (TOPK_CAP entries of 8 bytes
 // per query row).
 long buf_room(const TopkArgs& t) { return (long)t.B * t.H * t.Tq * TOPK_CAP * 8 / ((long)QB * buf_pitch(t) * 4); }
+// Keys of a head's first n rows (a padded sequence counted as a whole one).
+long keys_of(const TopkArgs& t, long n) {
+  if (!t.causal) return n * t.Tk;
+  const long off = t.q_offset, a = std::min(n, std::max(0L, -off)), b = std::min(n, std::max(a, t.Tk - off - 1));
+  return (b - a) * (a + b + 2 * off + 1) / 2 + (n - b) * t.Tk;
+}
+// D = 128, unsorted: whether the keys of rows that keep all of theirs decide.  The row kernel writes such a row
+// from one sweep, at half of this form's time a key, and spends some 256 keys' time more on each other row;
+// a workgroup's chain of tiles hides behind the others' work from 84 rows of full length to a CU on, 42 where no
+// row selects.  Rows of all keys or nearly all, us, row kernel and this form: 32 heads T = 1024 k = 1024
+// bf16 70 and 133, fp32 121 and 201; 64 heads T = 2048 k = 1024 651 and 695, k = 700 580 and 584;
+// 64 heads T = 640 k = 520 109 and 84, 128 heads 150 and 182; T = 600 k = 300, 128 heads 190 and 140.
+bool mostly_kept(const TopkArgs& t) {
+  const long kept = t.top_k >= t.Tk ? t.Tq : t.causal ? std::min<long>(t.Tq, std::max<long>(0, (long)t.top_k - t.q_offset)) : 0;
+  const long all = keys_of(t, kept), longest = t.causal ? std::min<long>(t.Tk, (long)t.Tq + t.q_offset) : t.Tk;
+  return all > 0 && all >= 512 * (t.Tq - kept) && (long)t.B * t.H * keys_of(t, t.Tq) >= (kept < t.Tq ? 84 : 42) * 256 * longest;
+}
 }  // namespace
 
 bool topk_buf_fits(const TopkArgs& a) {
   if (a.dump != nullptr || a.tl_list != nullptr || a.thr != nullptr) return false;
-  if (a.Tk > (a.D == DP ? (a.sort && a.top_k <= BUF_SORT ? 4096 : 2048) : BUF_MAXK)) return false;
+  const bool sorts = a.sort && a.top_k <= BUF_SORT;
+  if (a.Tk > (a.D == DP ? (sorts ? 4096 : 2048) : BUF_MAXK)) return false;
+  if (a.D == DP && !sorts && mostly_kept(a)) return false;
   // at most one pass more than whole row blocks take: a few rows of long heads stay on the row kernel
   const long blocks = (long)a.B * a.H * ((a.Tq + QB - 1) / QB);
   return buf_room(a) * ((buf_pitch(a) + 1023) / 1024 + 1) >= blocks;

@@ -78,3 +78,70 @@ def test_score_buffer_select(dev, dt, B, Tq, Tk, H, D, top_k, kind):
                         assert torch.equal(gs, vals)
                         assert (idx[b, h, r, n:] == 0).all()
                         assert top2[b, h, r, 0] == row.max()
+
+
+def _buffer_form(B, Tq, Tk, H, D, k, srt, causal, off):
+    """topk_buf.hip topk_buf_fits: whether a call takes this form or the row kernel."""
+    sorts = srt and k <= 512
+    if Tk > ((4096 if sorts else 2048) if D == 128 else 8192):
+        return False
+
+    def keys(n):
+        rows = torch.arange(n)
+        return int((rows + off + 1).clamp(0, Tk).sum()) if causal else n * Tk
+
+    if D == 128 and not sorts:
+        kept = Tq if k >= Tk else min(Tq, max(0, k - off)) if causal else 0
+        longest = min(Tk, Tq + off) if causal else Tk
+        if 0 < keys(kept) >= 512 * (Tq - kept) and B * H * keys(Tq) >= (84 if kept < Tq else 42) * 256 * longest:
+            return False
+    pitch = (Tk + 255) // 256 * 256 + 64
+    room = B * H * Tq * 512 * 8 // (64 * pitch * 4)
+    return room * ((pitch + 1023) // 1024 + 1) >= B * H * ((Tq + 63) // 64)
+
+
+def _keys(x):   # the order-preserving key of an fp32 score, -0 as +0
+    b = torch.where(x == 0, torch.zeros_like(x), x).contiguous().view(torch.int32).long() & 0xffffffff
+    return torch.where(b >= 2 ** 31, 2 ** 32 - 1 - b, b + 2 ** 31)
+
+
+def _check_form(dev, dt, B, Tq, Tk, H, D, top_k, kind, causal, srt, form):
+    """Every row against a stable sort of score_dump's keys, on the form that the rule names: the buffer form leaves
+    an unsorted row as one ascending run, the row kernel the keys of the cut's bin after the others."""
+    q, k = _inputs(torch.bfloat16 if dt == "bf16" else torch.float32, B, Tq, Tk, H, D, kind, dev)
+    off = max(0, Tk - Tq) if causal else 0
+    kk = min(top_k, Tk)
+    assert _buffer_form(B, Tq, Tk, H, D, kk, srt, causal, off) == form
+    dump = sgsa_amd.score_dump(q, k, 0, Tq, causal=causal, q_offset=off)
+    got = sgsa_amd.score_topk(q, k, top_k, causal=causal, q_offset=off, sorted=srt, fast=False, return_split=not srt)
+    idx, sc, top2, cnt = got[:4]
+    if not srt and kind == "random":
+        assert torch.equal(got[4], cnt) == form
+    nv = (torch.arange(Tq, device=dev) + off + 1).clamp(max=Tk) if causal else torch.full((Tq,), Tk, device=dev)
+    n = nv.clamp(max=kk)
+    assert torch.equal(cnt, n.int().expand(B, H, Tq))
+    valid = torch.arange(Tk, device=dev) < nv[:, None]
+    for h in range(H):   # by head: the sorts take 24 bytes a score
+        d = dump[:, h]
+        order = torch.sort(torch.where(valid, _keys(d), torch.full((), -1, device=dev)), dim=-1, descending=True, stable=True)[1][..., :kk]
+        used = torch.arange(kk, device=dev) < n[:, None]
+        gi, gs = idx[:, h].long(), sc[:, h]
+        if not srt:
+            big = torch.where(used, gi, torch.full((), Tk, device=dev)).sort(dim=-1)
+            gi, gs = big[0], gs.gather(-1, big[1])
+            order = torch.where(used, order, torch.full((), Tk, device=dev)).sort(dim=-1)[0]
+        want = d.gather(-1, order.clamp(max=Tk - 1))
+        u = used.expand(B, Tq, kk)
+        assert torch.equal(gi[u], order[u]), h
+        assert torch.equal(_keys(gs[u]), _keys(want[u])), h
+        assert (idx[:, h][~u] == 0).all()
+        best = torch.where(valid & ~d.isnan(), d, torch.full((), torch.finfo(torch.float32).min, device=dev)).amax(-1)
+        assert torch.equal(top2[:, h, :, 0], best)
+
+
+@pytest.mark.parametrize("dt", ["bf16", "fp32"])
+@pytest.mark.parametrize("H,T,top_k,causal,form", [(128, 640, 520, True, False), (64, 640, 520, True, True),
+                                                   (128, 640, 520, False, True), (96, 600, 300, True, True)])
+def test_mostly_kept_rows_take_the_row_kernel(dev, dt, H, T, top_k, causal, form):
+    print(f"score buffer form {dt} {H} {T} {top_k} {causal}", flush=True)
+    _check_form(dev, dt, 1, T, T, H, 128, top_k, "random", causal, False, form)

@@ -3,7 +3,10 @@ tiles, registers and LDS lists: key counts around 64, 256 and the 2048-, 4096- a
 8192-key register forms, more slots than the sorted list holds (512), bins that
 overflow it (mass ties), infinite scores, and dimensions and alignments that take
 the staged score kernel.  Indices and scores must equal the lowest-index top-k of
-the exact scores score_dump returns, bit for bit, sorted and unsorted."""
+the exact scores score_dump returns, bit for bit, sorted and unsorted.  The first
+list runs on whichever form the dispatch takes (its calls of few rows and many keys
+take the row kernel); FORMS names the form, which shows in an unsorted row's runs.
+NaN scores sort by their bits as the order key has them, a positive NaN above +inf."""
 
 import pytest
 import torch
@@ -39,6 +42,9 @@ def _inputs(dt, B, Tq, Tk, H, D, kind, dev):
         k[:, ::37] = 0.0
         k[:, ::37, :, 0] = 3e38
         q[..., 0] = torch.sign(q[..., 0]) * 1e3
+    if kind == "nan":   # keys whose scores are NaN
+        k = k.clone()
+        k[:, 3::41, :, D // 2] = float("nan")
     out = []
     for x in (q, k):
         buf = torch.empty(x.numel() + 1, dtype=dt, device=dev)
@@ -145,3 +151,33 @@ def _check_form(dev, dt, B, Tq, Tk, H, D, top_k, kind, causal, srt, form):
 def test_mostly_kept_rows_take_the_row_kernel(dev, dt, H, T, top_k, causal, form):
     print(f"score buffer form {dt} {H} {T} {top_k} {causal}", flush=True)
     _check_form(dev, dt, 1, T, T, H, 128, top_k, "random", causal, False, form)
+
+
+FORMS = [  # dtype, B, Tq, Tk, H, D, top_k, kind, the buffer form when sorted and when not
+    # the registers of a row: 1, 2, 4, 8, 16 and 32 vectors of 256 keys
+    ("bf16", 1, 100, 192, 2, 128, 1, "random", True, True), ("bf16", 1, 128, 257, 2, 128, 64, "random", True, True),
+    ("fp32", 2, 129, 600, 3, 64, 65, "random", True, True), ("bf16", 1, 200, 1100, 2, 128, 128, "random", True, True),
+    ("bf16", 1, 300, 2300, 2, 64, 129, "random", True, True), ("fp32", 1, 320, 4097, 2, 96, 257, "random", True, True),
+    ("bf16", 1, 640, 5000, 2, 40, 33, "random", True, True), ("fp32", 1, 640, 5000, 2, 64, 512, "random", True, True),
+    ("bf16", 1, 320, 8192, 2, 64, 700, "random", True, True),
+    # D = 128: the key limits of the sorted and unsorted calls, and lists that are too long to sort here
+    ("bf16", 1, 320, 4096, 2, 128, 65, "random", True, False), ("fp32", 1, 320, 4000, 2, 128, 512, "random", True, False),
+    ("bf16", 1, 320, 4097, 2, 128, 65, "random", False, False), ("bf16", 1, 300, 2049, 2, 128, 256, "random", True, False),
+    ("bf16", 1, 300, 2048, 2, 128, 513, "random", True, True), ("fp32", 1, 300, 2048, 2, 128, 600, "random", True, True),
+    # too few rows for a slab of the buffer
+    ("bf16", 1, 256, 8192, 2, 64, 33, "random", False, False), ("bf16", 1, 70, 4096, 2, 128, 65, "random", False, False),
+    # scores that no histogram separates, and those that are no numbers
+    ("bf16", 1, 640, 5000, 2, 64, 300, "tied", True, True), ("fp32", 1, 640, 5000, 2, 64, 600, "equal", True, True),
+    ("bf16", 1, 320, 4096, 2, 128, 500, "equal", True, False), ("fp32", 1, 320, 3000, 2, 64, 400, "infinite", True, True),
+    ("bf16", 1, 320, 4096, 2, 128, 300, "infinite", True, False), ("bf16", 1, 130, 700, 2, 128, 90, "nan", True, True),
+    ("bf16", 1, 130, 700, 2, 128, 600, "nan", True, True), ("fp32", 1, 320, 4100, 2, 64, 64, "nan", True, True),
+    ("fp32", 1, 130, 300, 2, 40, 3, "nan", True, True),
+]
+
+
+@pytest.mark.parametrize("dt,B,Tq,Tk,H,D,top_k,kind,srt,uns", FORMS)
+def test_select_forms(dev, dt, B, Tq, Tk, H, D, top_k, kind, srt, uns):
+    print(f"score buffer forms {dt} {B} {Tq} {Tk} {H} {D} {top_k} {kind}", flush=True)
+    for causal in (True, False):
+        for s, form in ((True, srt), (False, uns)):
+            _check_form(dev, dt, B, Tq, Tk, H, D, top_k, kind, causal, s, form)

@@ -18,16 +18,18 @@ pytestmark = pytest.mark.gpu
 import sgsa_amd  # noqa: E402  (pure Python; the HIP library loads on first call and raises if missing)
 
 
-def _qkv(B, T, H, D, dt, seed, dup=False):
+def _qkv(B, T, H, D, dt, seed, dup=False, ints=False):
     g = torch.Generator().manual_seed(seed)
     x = [torch.randn(B, T, H, D, generator=g) for _ in range(3)]
+    if ints:   # q and k of small whole numbers: every sum is exact in fp32, and many scores tie
+        x[:2] = [t.round().clamp(-2, 2) for t in x[:2]]
     if dup:   # every key equal: all scores of a row tie
         x[1] = x[1][:, :1].expand(B, T, H, D).contiguous()
     return [t.to(dt).float() for t in x]
 
 
-def _check(dev, B, T, H, D, dt, top_k, bs, tb, mode, causal=True, seed=0, dup=False, am=None):
-    q, k, v = _qkv(B, T, H, D, dt, seed, dup)
+def _check(dev, B, T, H, D, dt, top_k, bs, tb, mode, causal=True, seed=0, dup=False, am=None, ints=False):
+    q, k, v = _qkv(B, T, H, D, dt, seed, dup, ints)
     ref = O.block_retrieval(q, k, v, top_k, bs, tb, mode=mode, causal=causal, attention_mask=am)
     got = sgsa_amd.block_retrieve(q.to(dev, dt), k.to(dev, dt), v.to(dev, dt), top_k, bs, tb, mode=mode,
                                   causal=causal, return_block_scores=True,
@@ -58,6 +60,23 @@ def _check(dev, B, T, H, D, dt, top_k, bs, tb, mode, causal=True, seed=0, dup=Fa
                                            (33, 32, 4, 48), (300, 16, 3, 20), (260, 48, 2, 30)])
 def test_block_modes_match_oracle(dev, dt, mode, T, bs, tb, top_k):
     _check(dev, 2, T, 3, 64, dt, top_k, bs, tb, mode, seed=T + bs)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,bs,tb,top_k,masked", [
+    (560, 1, 540, 30, False),      # 1 .. 540 candidates, one more per row: every size of the register sort, and LDS
+    (600, 64, 4, 300, False),      # up to 256, fewer than the slots
+    (330, 1, 257, 40, False), (640, 64, 8, 100, False),    # 257; 512
+    (700, 64, 9, 16, False), (1150, 64, 16, 700, False),   # 576 and 1024 in LDS, fewer slots than candidates
+    (1150, 1, 1000, 1100, False),  # 1000 in LDS, more slots
+    (700, 64, 9, 600, True)])
+def test_block_token_candidate_counts(dev, dt, T, bs, tb, top_k, masked):
+    """block_cand_kernel's sort of a row's candidates at its register sizes (64, 128, 256, 512) and in LDS past
+    them, with ties between candidates (the lowest key first)."""
+    B = 3 if masked else 1
+    print(f"block candidates {dt} T={T} bs={bs} tb={tb} k={top_k} masked={masked}", flush=True)
+    _check(dev, B, T, 1, 64, dt, top_k, bs, tb, "block_token", seed=T + tb, am=_pad(B, T) if masked else None,
+           ints=True)
 
 
 @pytest.mark.parametrize("mode", ["block_token", "block_only"])

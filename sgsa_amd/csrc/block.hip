@@ -39,12 +39,6 @@ __device__ __forceinline__ float block_score(float acc, float mscale) {
   return acc * mscale + 0.0f;
 }
 
-__device__ __forceinline__ void wave_sync_lds() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // ---- padding masks ----------------------------------------------------------
 // One 1024-thread workgroup per batch b, over the positions in tiles of 1024:
 // pass 1 writes pc[t] = valid keys before t (pc[T] = all of them), perm[pc[t]]
@@ -865,7 +859,7 @@ __global__ __launch_bounds__(64) void block_cand_kernel(BlockArgs a, float mscal
     run += __shfl(inc, 63, 64);
   }
   const int ncand = run;
-  wave_sync_lds();
+  wave_lds_sync();
 
   auto key_of = [&](int c) {
     int lo = 0, hi = kqb - 1;
@@ -998,7 +992,7 @@ __global__ __launch_bounds__(64) void block_cand_kernel(BlockArgs a, float mscal
     os[i] = key_to_f32(ord);
     ov[i] = 1;
   };
-  wave_sync_lds();
+  wave_lds_sync();
   if (ncand <= 512) {
     auto sort = [&](auto ns) __attribute__((always_inline)) {
       constexpr int NS = decltype(ns)::value;
@@ -1027,7 +1021,7 @@ __global__ __launch_bounds__(64) void block_cand_kernel(BlockArgs a, float mscal
     int npad = 1;
     while (npad < ncand) npad <<= 1;
     for (int c = ncand + lane; c < npad; c += 64) keys[c] = ~0ull;
-    wave_sync_lds();
+    wave_lds_sync();
     for (int span = 2; span <= npad; span <<= 1) {
       for (int j = span >> 1; j > 0; j >>= 1) {
         for (int i = lane; i < npad; i += 64) {
@@ -1040,7 +1034,7 @@ __global__ __launch_bounds__(64) void block_cand_kernel(BlockArgs a, float mscal
             }
           }
         }
-        wave_sync_lds();
+        wave_lds_sync();
       }
     }
     for (int i = lane; i < nv; i += 64) put(i, (uint32_t)keys[i], ~(uint32_t)(keys[i] >> 32));

@@ -137,12 +137,6 @@ __device__ __forceinline__ void mm_col(f4 (&acc)[NR], const float* a, const f4& 
   }
 }
 
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // 16x16 LDS tiles (row-major, pitch TLP): acc + X Y, and a store from the accumulator layout.
 __device__ __forceinline__ f4 tile_mm(const float* X, const float* Y, f4 acc, int lr, int lg) {
   const f4 x = *reinterpret_cast<const f4*>(X + lr * TLP + 4 * lg);

@@ -117,6 +117,14 @@ __device__ __forceinline__ f4 f4_zero() {
 __device__ __forceinline__ int lane_id() { return threadIdx.x & 63; }
 __device__ __forceinline__ int wave_id() { return threadIdx.x >> 6; }
 
+// Between a wave's LDS stores and its lanes' reads of each other's words (a wave's LDS accesses stay in order; this
+// keeps the compiler's order).
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // x of lane ^ M in VALU instructions: DPP within a row of 16 lanes, the row and half swaps across
 // rows.  A shuffle through LDS takes an address, a trip to LDS and a wait per
 // word: block retrieval's gather (131072 rows of 64 slots, some 20 reductions each) 214 us with those,

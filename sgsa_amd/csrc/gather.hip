@@ -296,9 +296,7 @@ __device__ __forceinline__ bool gather_slots_mx(const GatherArgs& a, int kq, con
     L.part[0][lane] = (uint16_t)(__float_as_uint(wgt) >> 16);
     L.part[1][lane] = (uint16_t)(__float_as_uint(w1) >> 16);
     L.part[2][lane] = (uint16_t)(__float_as_uint(w2) >> 16);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_lds_sync();
     const int nstep = min(64, kq - base);
 #pragma unroll 1
     for (int it = 0; it * rpi * 4 < nstep; ++it) {

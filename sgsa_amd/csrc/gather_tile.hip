@@ -44,12 +44,6 @@ constexpr int KT = 64;
 constexpr int DP = 128;
 constexpr int PT = KT + 8;   // pitch (bf16) of the transposed K/V tiles and of P
 
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 __device__ __forceinline__ bf16x8 as_bf8(uint4 u) { return __builtin_bit_cast(bf16x8, u); }
 
 // One ascending run of a row's slot list.  Lane quarter lg holds positions

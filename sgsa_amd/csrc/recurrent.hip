@@ -53,7 +53,7 @@ constexpr int TC = 8;   // tokens of a chunk
 // Sum over the aligned group of N = 4 or 8 lanes, in every lane, in sum_chains' order: quad_perm ^1,
 // ^2, then row_half_mirror.  With 4 groups the other four chains are zeros.
 template <int N>
-__device__ __forceinline__ float sum_groups(float x) {
+__device__ __forceinline__ float sum_row_groups(float x) {
   x += __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(x), 0xb1, 0xf, 0xf, true));
   x += __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(x), 0x4e, 0xf, 0xf, true));
   if constexpr (N == 8)
@@ -185,8 +185,8 @@ __global__ __launch_bounds__(256) void recurrent_seq_kernel(RecurrentArgs a, int
       // the next one's overlap (a loop that breaks at T: 8 to 15% slower with up to 128 heads).
       const uint32_t live = (uint32_t)((t0 + t - T) >> 31);   // all bits, or none
       auto kept = [&](float x) __attribute__((always_inline)) { return __uint_as_float(__float_as_uint(x) & live); };
-      const float dl = kept(bet * (val[buf][t][0][cl] - sum_groups<NRG>(pk)));
-      const float ds = SP ? kept(alp * (val[buf][t][NVAL - 1][cl] - sum_groups<NRG>(ph))) : 0.f;
+      const float dl = kept(bet * (val[buf][t][0][cl] - sum_row_groups<NRG>(pk)));
+      const float ds = SP ? kept(alp * (val[buf][t][NVAL - 1][cl] - sum_row_groups<NRG>(ph))) : 0.f;
       // rank-1 writes, then the readout o = S^T q
       float po = 0.f;
 #pragma unroll
@@ -195,7 +195,7 @@ __global__ __launch_bounds__(256) void recurrent_seq_kernel(RecurrentArgs a, int
         if constexpr (SP) S[r] = fmaf(h4[r / 4][r % 4], ds, S[r]);
         po = fmaf(S[r], q4[r / 4][r % 4], po);
       }
-      const float o = sum_groups<NRG>(po);
+      const float o = sum_row_groups<NRG>(po);
       out[t / NRG] = rg == t % NRG ? o : out[t / NRG];
     }
 #pragma unroll

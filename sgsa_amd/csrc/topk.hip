@@ -122,12 +122,6 @@ __device__ __forceinline__ float bin_lower_edge(int bt, float iw, float bc = BIN
   return key_to_f32(hi);
 }
 
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Over 256 counts laid out as lane l <-> bins 255-4l .. 252-4l (descending),
 // finds the bin holding the `need`-th largest element.  Wave-uniform results.
 __device__ __forceinline__ void find_bin(const uint32_t (&c)[4], int lane, uint32_t need, int& bin, uint32_t& above,

@@ -66,12 +66,6 @@ __device__ __forceinline__ int block_keys(const TopkArgs& t, int r0) {
   return t.causal ? min(t.Tk, min(t.Tq, r0 + QB) + t.q_offset) : t.Tk;
 }
 
-__device__ __forceinline__ void lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // bf16, D = 32 NKS, 16-byte rows: wave w scores keys [64w, 64w + 64) of the workgroup's 256
 // against its 64 rows; keys are the MFMA's A operand and rows its B operand, so a lane holds four
 // consecutive keys of one row.
@@ -119,11 +113,11 @@ __global__ __launch_bounds__(256) void buf_score_kernel(BufArgs a, float mscale)
     }
 #pragma unroll
     for (int kg = 0; kg < 4; ++kg) *reinterpret_cast<f4*>(ts + lr * TP + 16 * kg + 4 * lg) = score_of(c[kg], mscale);
-    lds_sync();
+    wave_lds_sync();
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       *reinterpret_cast<f4*>(out + (long)(16 * g + 4 * j) * a.pitch) = *reinterpret_cast<const f4*>(ts + (4 * j + lg) * TP + 4 * lr);
-    lds_sync();
+    wave_lds_sync();
   }
 }
 
@@ -341,14 +335,14 @@ __global__ __launch_bounds__(256) void buf_select_kernel(BufArgs a) {
     uint32_t bin = 0;
     if (inv <= FLT_MAX && fabsf(lo * inv) <= 4194304.f) {
       *reinterpret_cast<uint4*>(hist + 4 * lane) = make_uint4(0, 0, 0, 0);
-      lds_sync();
+      wave_lds_sync();
 #pragma unroll
       for (int i = 0; i < NV; ++i) {
         if (256 * i >= nv) continue;
 #pragma unroll
         for (int e = 0; e < 4; ++e) atomicAdd(&hist[bin_of(v[i][e]) & 255u], 1u);   // -inf: bin 0
       }
-      lds_sync();
+      wave_lds_sync();
       uint32_t c[4];
 #pragma unroll
       for (int q = 0; q < 4; ++q) c[q] = hist[255 - 4 * lane - q];
@@ -386,7 +380,7 @@ __global__ __launch_bounds__(256) void buf_select_kernel(BufArgs a) {
           }
         }
       }
-      lds_sync();
+      wave_lds_sync();
       auto search = [&](auto NC) __attribute__((always_inline)) {
         constexpr int N = decltype(NC)::value;
         uint32_t ck[N];
@@ -405,7 +399,7 @@ __global__ __launch_bounds__(256) void buf_select_kernel(BufArgs a) {
       };
       if (cnt <= 64) search(std::integral_constant<int, 1>{});
       else search(std::integral_constant<int, CAP / 64>{});
-      lds_sync();
+      wave_lds_sync();
     } else {
       keys = true;
     }
@@ -484,7 +478,7 @@ __global__ __launch_bounds__(256) void buf_select_kernel(BufArgs a) {
     }
   }
   if (!lds) return;
-  lds_sync();
+  wave_lds_sync();
   const bool sort = t.sort != 0;
   if (kq <= 64) put_row<1>(list, kq, sort, oi, os, lane);
   else if (kq <= 128) put_row<2>(list, kq, sort, oi, os, lane);

@@ -978,7 +978,8 @@ __global__ __launch_bounds__(64) void block_cand_kernel(BlockArgs a, float mscal
   }
 
   // the candidates by (score desc, key asc): up to 512 in registers, more in LDS (131072 rows of 64
-  // candidates: 287 us all in LDS, 281; the reads of the candidates' keys, 2.1 GB, bound both)
+  // candidates: 287 us all in LDS, 281 so: a wave waits four fifths of its time on its row's chain of loads
+  // (counters, as VALU issue 47%), and the sort is not what it waits for)
   int mc = max(1, mcl);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) mc = max(mc, __shfl_xor(mc, o, 64));

@@ -199,8 +199,8 @@ __global__ __launch_bounds__(64 * (M / 16), sizeof(X) == 2 || DP == 64 ? 4 : 2) 
 // V's columns of sample tile w, then a share of the column tiles of Phi and Pm, which use every
 // read of the staged V twice.
 //
-// fp32 MFMA work, 664 products of 32 cycles per wave at M = DP = 128; the staged operand is read
-// once for both maps.  bf16, B=4 T=4096 H=8 D=128: 235 us, 60 TFLOP/s, against 539 us for 16x16
+// fp32 MFMA work, 656 products of 32 cycles per wave at M = DP = 128; the staged operand is read
+// once for both maps.  bf16, B=4 T=4096 H=8 D=128: 235 us, 94 TFLOP/s, against 539 us for 16x16
 // tiles that each read both operands from LDS.
 // ---------------------------------------------------------------------------
 template <typename X, int M, int DP, bool FULL>
@@ -299,11 +299,12 @@ __global__ __launch_bounds__(4 * M) void chunk_maps_kernel(ChunkArgs f, const fl
 // one MFMA chain per wave over its own 16 rows of Phi, loaded straight into
 // registers one step ahead, and one barrier to exchange x through LDS.
 //
-// A step is latency: 32 dependent MFMAs at DP = 128 and a barrier, about 2.9 us.  That is less
-// than a quarter of a step with a head's whole state in one workgroup (12 us), which is why the
-// chunks are not also split into segments: at B=4 T=4096 H=8 D=128 (64 chunks) 197 us against
-// 340 us for a segmented scan in three passes, and about even at T = 32768 with 16 heads, by
-// the steps' times (512 of these, 112 of the segmented form's).
+// A step takes 2.7 to 3.1 us at DP = 128, of which the two waves of a SIMD issue MFMAs (two chains of 16
+// each) for 0.85; the rest is the wait for Phi, 64 KB per workgroup and step loaded one step ahead, and the
+// barrier.  That is a quarter of a step with a head's whole state in one workgroup (12 us), which is why the
+// chunks are not also split into segments: at B=4 T=4096 H=8 D=128 (64 chunks) 197 us against 340 us for
+// a segmented scan in three passes.  Longest, 512 chunks of 16 heads: 1.40 ms forward and 1.23 back, against 1.38
+// and 1.42 segmented; the whole backward of one head at T = 32768 2.72 against 3.84 ms.
 // ---------------------------------------------------------------------------
 template <int DP, bool TR>
 __global__ __launch_bounds__(4 * DP) void chunk_scan_kernel(const float* __restrict__ phi, const float* __restrict__ y,

@@ -338,7 +338,12 @@ __global__ __launch_bounds__(64 * K3W) void chunk_inv_bf16(const bf16_t* __restr
 // segments of 8 chunks and half as many workgroups, then so: 16 heads T = 4096 241 -> 185 us, 2048
 // 212 -> 139, 1024 201 -> 121, 576 134 -> 95; one head T = 4096 210 -> 148; 200 heads T = 2048 (one
 // segment instead of two that do not fit in one round) 969 -> 551.  Eight chunks or fewer stay in one
-// segment: 16 heads T = 512 100 us, in two segments 112.
+// segment: 16 heads T = 512 100 us, in two segments 112.  D < 128 has two workgroups of half the work per
+// segment in the maps, and gains the same: D = 64, 16 heads T = 4096 212 -> 194, 1024 170 -> 104, one head 4096
+// 181 -> 132, 208 heads 1024 547 -> 293; none of 116 shapes was slower.
+// The segment starts come from S = Phi S + P, so with other segments the bf16 roundings of the carried state's
+// products fall elsewhere and the output's last bits change; its error against 64 bits does not (26 shapes, 22
+// with other segments than before: by 2e-5 of the error in the output, 4e-4 in the state, of either sign).
 inline int seg_count(int BH, int NT) {
   int g = 256 / BH;
   g = g < 32 ? g : 32;

@@ -189,12 +189,12 @@ __global__ __launch_bounds__(4 * M) void chunk_bwd_pre_kernel(ChunkBwdArgs a, co
 // matrices the waves share at a time: S and B = nu - diag(e^l_tau) kappa S; S and G; S and dR; R and
 // kappa; X, Y and kappa.
 //
-// fp32 MFMA work: about 35 MFLOP per chunk at M = DP = 128 (triangular products cut at the tile,
-// dT as one product) where the direct form of the gradient takes 69, and no intermediate leaves
-// the CU.  bf16, B=4 T=4096 H=8 D=128 (2048 chunks): 968 us, 74 TFLOP/s, against 3876 us with
-// 16x16 tiles and R, dR, dW, Z, dA, X in a per-chunk workspace.  What remains over the 470 us of
-// MFMA time is one workgroup per CU at two waves per SIMD: the barriers between phases and the
-// LDS reads ahead of each product show.
+// fp32 MFMA work: 39 MFLOP per chunk at M = DP = 128 (triangular products cut at the tile, dT as one
+// product) where the direct form of the gradient takes 69, and no intermediate leaves the CU.  bf16, B=4
+// T=4096 H=8 D=128 (2048 chunks): 910 us, 87 TFLOP/s, against 3876 us with 16x16 tiles and R, dR, dW, Z,
+// dA, X in a per-chunk workspace (968 us with the gate gradients in LDS atomics).  What remains over the 506 us
+// of MFMA time is one workgroup per CU at two waves per SIMD: the barriers between phases and the LDS
+// reads ahead of each product show.
 template <typename X, int M, int DP, bool FULL>
 __global__ __launch_bounds__(64 * (M / 16)) void chunk_bwd_grad_kernel(ChunkBwdArgs a,
                                                                        const float* __restrict__ X1g,

@@ -127,7 +127,7 @@ __device__ __forceinline__ void wave_lds_sync() {
 
 // x of lane ^ M in VALU instructions: DPP within a row of 16 lanes, the row and half swaps across
 // rows.  A shuffle through LDS takes an address, a trip to LDS and a wait per
-// word: block retrieval's gather (131072 rows of 64 slots, some 20 reductions each) 214 us with those,
+// word: block retrieval's gather (131072 rows of 16 slots, some 20 reductions each) 214 us with those,
 // 204 so.
 template <int M>
 __device__ __forceinline__ uint32_t lane_xor(uint32_t x, int lane) {

@@ -213,6 +213,8 @@ __device__ __forceinline__ void gather_slots(const GatherArgs& a, int s0, int s1
 // slots: value rows 295 -> 183 us, key and value rows 413 -> 318; 64 slots 120 -> 81 and 158 -> 122; what
 // bounds it now is the rows' delivery from L2 (8.6 GB at 27 TB/s with both).  Four or five waves to a
 // SIMD (launch bounds) before more loads in flight in each: eight slots a step without key rows 206.
+// Rows of 16 slots (block retrieval's) are bound by VALU issue instead, 808 instructions a row by the
+// counters, most of them the epilogue's.
 // A lane group of LPR lanes (LPR >= 4, a multiple of the block) takes four consecutive slots a step;
 // the slots' row offsets and weight parts pass through LDS, one write per slot and one read per step.
 // A part of 0 times an inf is a NaN that the plain product does not have: the caller takes the plain

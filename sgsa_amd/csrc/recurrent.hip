@@ -42,8 +42,8 @@ __global__ __launch_bounds__(256) void recurrent_kernel(RecurrentArgs a) {
 // a chunk's outputs leave in one or two stores.
 //
 // Bound by the VALU at two waves per SIMD (16 rows x 6 operations a token and lane) and by the
-// chain of a token at one.  T = 256, bf16 D = 128 with the sparse write, before and after: 128
-// heads 341 -> 165 us, one head 302 -> 113, 512 heads 1068 -> 495; D = 64, 512 heads 1001 -> 168.
+// chain of a token at one.  T = 256, bf16 D = 128 with the sparse write, a call by events, before and after:
+// 128 heads 338 -> 152 us, one head 300 -> 112, 512 heads 1060 -> 479; D = 64, 512 heads 1000 -> 164.
 // Two columns a lane (half the LDS reads) were slower: 236 us at 128 heads, 192 at one.
 // ---------------------------------------------------------------------------
 namespace {
@@ -226,7 +226,7 @@ static void launch_seq_t(const RecurrentArgs& a, hipStream_t st) {
 
 template <typename X, bool SP>
 static void launch_rec_t(const RecurrentArgs& a, hipStream_t st) {
-  // from 4 tokens on (512 heads of 128, bf16: T = 2 31.9 us here and 36.3 there, T = 4 40.0 and 35.2)
+  // from 4 tokens on (512 heads of 128, bf16, one-token form and this one: T = 2 31.9 us and 36.3, T = 4 40.0 and 35.2)
   if (a.T >= 4) {
     if (a.D <= 64) launch_seq_t<X, SP, 4>(a, st);
     else launch_seq_t<X, SP, 8>(a, st);

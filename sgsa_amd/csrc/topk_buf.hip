@@ -17,8 +17,10 @@
 // The buffer is the row kernel's own workspace (TOPK_CAP 8-byte candidates per
 // row, 4 KB); longer rows take several passes over slabs of row blocks.
 //
-// What bounds it: the buffer's bytes (T = 4096 with 16 heads: 0.55 GB written and read, scores 215
-// us, select 260 us, its sort 90 us) and, in the select, about 20 VALU instructions a score.
+// What bounds it, T = 4096 with 16 heads, k = 256: the scores the buffer's bytes (0.55 GB written, 215 us);
+// the select VALU issue (92% busy by the counters; 260 us, its sort 78 more): 2620 instructions a row of 2048
+// scores on average, some 600 of them the sort's, and one LDS atomic a score, whose bank conflicts take 10%
+// of the CUs' cycles.
 // B=1 H=16, score_topk before and after, us: bf16 D=128 T=1024 k=64 unsorted 128 -> 54, sorted
 // 171 -> 58; T=2048 k=128 207 -> 129, 319 -> 145; T=4096 k=256 479 -> 432, 806 -> 524 (with 128
 // heads 3013 -> 3132 unsorted, 3749 -> 3228 sorted); T=8192 1535 -> 2263, 2184 -> 2437.  D=64

@@ -573,13 +573,21 @@ def run_backward(args) -> int:
         log("backward: non-finite gradient")
         return 1
     log(f"native backward ms/call {ms:.3f}")
-    # fp32 MFMA multiply-adds per chunk-head (M = 2L samples with the sparse write, L tokens, d dims)
+    # fp32 MFMA work per chunk-head as the kernels issue it, in products of 16x16x16 tiles (M = 2L samples with the
+    # sparse write, L tokens, d dims; bf16 inputs: the Gram runs on bf16 MFMA and is not counted)
     M, L, d = 128, 64, 128
-    mac = (M * M * d + M ** 3 // 3                                       # intra: Gram, (I+T)^-1
-           + M * M * d + 2 * d * d * M                                   # maps: A^T kappa, Phi, Pm
-           + 2 * d ** 3                                                  # the two scans, one step each
-           + L * M * d + d * d * L + M * d * L + M * M * d + d * d * M   # pre: P, Q^T dO, P^T dO, A^T X1, kappa^T
-           + 17_500_000)                                                 # gradient kernel (triangles cut at the tile)
+    nb, lt, rt = M // 16, L // 16, d // 16
+    low = nb * (nb + 1) // 2                                 # sample by sample, on and below the diagonal
+    pairs = 2 * sum(range(2, nb + 1, 2))                     # the same in pairs of tiles
+    ptok = (M // L) * lt * (lt + 1) // 2                     # token by sample, tau <= t
+    tiles = (sum(nb // (2 * n) * n * n * (n + 1) for n in (1, 2, 4))     # intra: (I+T)^-1 by doubling
+             + low * rt + 2 * nb * rt * rt                               # maps: A^T kappa; Phi, Pm
+             + 2 * rt ** 3                                               # the two scans, one step each
+             + 2 * ptok * rt + lt * rt * rt + low * rt + nb * rt * rt    # pre: P, P^T dO; Q^T dO; A^T X1; kappa^T
+             # gradient: kappa S, kappa G, R G^T, dnu S^T; dO S^T; R, dnu, X kappa, X^T kappa; dT, kappa kappa^T;
+             # q kappa^T, dP, Y^T Q, Y kappa
+             + 4 * nb * rt * rt + lt * rt * rt + 4 * low * rt + 2 * pairs * rt + 4 * ptok * rt)
+    mac = 4096 * tiles
     nchunks = B * H * ((T + 63) // 64)
     flops = 2.0 * mac * nchunks
     torch_ms = None

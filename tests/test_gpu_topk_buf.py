@@ -166,6 +166,9 @@ FORMS = [  # dtype, B, Tq, Tk, H, D, top_k, kind, the buffer form when sorted an
     ("bf16", 1, 300, 2048, 2, 128, 513, "random", True, True), ("fp32", 1, 300, 2048, 2, 128, 600, "random", True, True),
     # too few rows for a slab of the buffer
     ("bf16", 1, 256, 8192, 2, 64, 33, "random", False, False), ("bf16", 1, 70, 4096, 2, 128, 65, "random", False, False),
+    # and the row kernel's sort of 256 and 512 slots in registers, and of more in LDS
+    ("bf16", 1, 70, 4500, 2, 128, 256, "random", False, False), ("fp32", 1, 70, 4500, 2, 128, 512, "random", False, False),
+    ("bf16", 1, 70, 4500, 2, 128, 513, "random", False, False),
     # scores that no histogram separates, and those that are no numbers
     ("bf16", 1, 640, 5000, 2, 64, 300, "tied", True, True), ("fp32", 1, 640, 5000, 2, 64, 600, "equal", True, True),
     ("bf16", 1, 320, 4096, 2, 128, 500, "equal", True, False), ("fp32", 1, 320, 3000, 2, 64, 400, "infinite", True, True),
